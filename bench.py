@@ -208,9 +208,11 @@ def plain_config(name, args, with_cpu=True):
     log(f"[bench] {name}: {'fixed' if args.shape else 'tuned'} shape {shape}")
     # direct launches of the same shape, for per-kernel HIP-event timings
     sort_bit = ptamd.PT_FLAG_MATERIAL_SORT if tune.material_sort else 0
-    direct = scene.render_params(flags=(info.flags & ~ptamd.PT_FLAG_MATERIAL_SORT) | sort_bit,
+    direct = scene.render_params(flags=(info.flags & ~ptamd.PT_FLAG_MATERIAL_SORT) | sort_bit | ptamd.PT_FLAG_DIRECT,
                                  frames_per_batch=tune.frames_per_batch)
-    tuned = direct if args.shape else scene.render_params(flags=info.flags | ptamd.PT_FLAG_TUNED)
+    tuned = scene.render_params(flags=info.flags | ptamd.PT_FLAG_TUNED)
+    if args.shape:
+        tuned = scene.render_params(flags=direct.flags & ~ptamd.PT_FLAG_DIRECT, frames_per_batch=tune.frames_per_batch)
     # traversal-counting pass (identical rays: the render is deterministic)
     cst = ctx.render(scene.render_params(flags=(info.flags & ~ptamd.PT_FLAG_MATERIAL_SORT) | sort_bit |
                                          ptamd.PT_FLAG_COUNT_TRAVERSAL, frames_per_batch=tune.frames_per_batch), 0, spp)

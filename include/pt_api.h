@@ -111,7 +111,8 @@ typedef int32_t pt_status;
 #define PT_FLAG_TUNED 0x40u          /* use pt_autotune's batch size, sort
                                         and graph choice when it matches     */
 #define PT_FLAG_DIRECT 0x80u         /* launch directly even where the tuned
-                                        shape replays graphs: per-kernel
+                                        shape replays graphs, and every bounce
+                                        in launches of its own: per-kernel
                                         times in the stats (extend_ms,
                                         shade_ms)                            */
 
@@ -296,7 +297,9 @@ typedef struct pt_render_stats {
   double gpu_ms;            /* render wall time on the stream (events)      */
   double extend_ms;         /* summed closest-hit kernel time               */
   double shade_ms;          /* summed shading kernel time (hit and miss
-                               programs, shadow rays, continuation)        */
+                               programs, shadow rays, continuation); without
+                               PT_FLAG_DIRECT also the one launch that runs
+                               a batch's last bounces whole                */
   uint32_t extend_launches;
   uint32_t shade_launches;
   uint64_t nan_paths;       /* paths whose color() had a NaN channel, which

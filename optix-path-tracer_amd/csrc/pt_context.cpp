@@ -258,6 +258,17 @@ int grid_for(uint64_t n) {
   return (int)std::max<uint64_t>(1, std::min<uint64_t>((n + BLOCK - 1) / BLOCK, cap));
 }
 
+// First bounce of the one launch that runs all the bounces left (SH_TAIL),
+// for a batch of n paths.  Its waves trace lock-step and unsorted, so it pays
+// from where a wave holds few paths: measured with 1, 2, 3, 4, 6 and 8 (and a
+// launch per kernel and bounce), 4 k paths of the Cornell box 339, 367, 389,
+// 401, 420, 458 (526) us; 1.0 M of the next-week scene 5.7, 4.9, 4.1, 3.9,
+// 4.4, 4.7 (10.5) ms; 1.7 M of the sphere scene 1.8, 1.8, 1.9, 2.0, 2.3, 2.5
+// (4.3) ms; 2.1 M of the mesh scene 4.2, 4.0, 4.6, 4.9, 5.4, 5.7 (6.0) ms;
+// 134 M of 16 scenes 70.7, 66.4, 67.0, 67.8, 67.6, 67.2 (70.0) ms; 199 M of
+// the mesh scene 85.1, 76.0, 74.6, 72.5, 71.9, 72.5 (73.3) ms.
+uint32_t tail_depth(uint64_t n) { return n < (1u << 18) ? 1u : n < (1u << 23) ? 3u : 4u; }
+
 // an odd stride near 0.618 n that is coprime to n (a full-period
 // multiplicative order of 0..n-1)
 uint32_t golden_stride(uint32_t n) {
@@ -1224,10 +1235,25 @@ pt_status pt_render(pt_context* c, const pt_render_params* rp, uint32_t frame_be
   hipEvent_t t_begin = want_stats ? mark() : nullptr;
   DevPaths& P = c->paths;
   const int matset = shade_material_set(c->mat_types);
-  // one batch: camera rays, the bounce loop, the paths that outlived it
+  // one batch: camera rays, the bounce loop, the paths that outlived it;
+  // from bounce `tail` on one launch does all three
   auto enqueue_batch = [&](uint32_t nslots, int grid, bool events) {
     int in = 0, out = 1;
+    // with the radiance cache: not before the queries are asked, and not in
+    // sorted batches (the sort's order is that of the training records)
+    uint32_t tail = tail_depth(nslots);
+    if (rc.flags & PT_FLAG_RADIANCE_CACHE) {
+      if (rc.cache.query_depth < rp->max_depth) tail = std::max(tail, rc.cache.query_depth + 1);
+      if (sort) tail = 0xFFFFFFFFu;
+    }
+    if (count_trav || (rp->flags & PT_FLAG_DIRECT)) tail = 0xFFFFFFFFu;
     for (uint32_t depth = 0; depth < rp->max_depth; depth++) {
+      if (depth == tail) {
+        hipEvent_t a = events ? mark() : nullptr;
+        launch_tail(c->dsc, P, in, out, depth, rc, matset, c->spill, c->stats, grid, c->stream);
+        if (events) sh_ev.push_back({a, mark()});
+        return;
+      }
       hipEvent_t a = events ? mark() : nullptr;
       // depth 0 starts the camera paths in the same launch
       // material sort from the first bounce on: a wave's camera hits are
@@ -1853,7 +1879,15 @@ pt_status render_batch_shaped(pt_context* const* ctxs, const pt_render_params* p
       const BatchStart bs{B->d_rcs, B->d_item_off + k0, B->d_item_scene + k0, B->d_item_frame + k0,
                           (uint32_t)(k1 - k0)};
       int in = 0, o = 1;
+      const uint32_t tail = (count_trav || (params[0].flags & PT_FLAG_DIRECT)) ? 0xFFFFFFFFu : tail_depth(nslots);
       for (uint32_t depth = 0; depth < max_depth; depth++) {
+        if (depth == tail) {
+          hipEvent_t a = kernel_events ? mark() : nullptr;
+          launch_tail(B->dsc, P, in, o, depth, rc0, matset, B->spill, B->stats, grid, B->stream, B->d_scenes,
+                      B->d_rcs, env, ext);
+          if (kernel_events) sh_ev.push_back({a, mark()});
+          break;
+        }
         const bool sd = sort && depth > 0;  // from the first bounce on, as in pt_render
         hipEvent_t a = kernel_events ? mark() : nullptr;
         launch_extend(B->dsc, P, in, depth == 0 ? 1e-6f : 1e-3f, B->spill, B->stats, count_trav, sd, grid,
@@ -1866,7 +1900,7 @@ pt_status render_batch_shaped(pt_context* const* ctxs, const pt_render_params* p
         if (kernel_events) sh_ev.push_back({a2, mark()});
         std::swap(in, o);
       }
-      launch_exhausted(P, in, B->stats, grid, B->stream);
+      if (tail >= max_depth) launch_exhausted(P, in, B->stats, grid, B->stream);
       for (size_t k = k0; k < k1;) {
         size_t e = k;
         while (e < k1 && scene[e] == scene[k]) e++;

@@ -63,6 +63,13 @@ void launch_shade(const DevScene& sc, const DevPaths& P, int in, bool sorted, in
                   const RenderConsts& rc, int matset, bool count, uint2* spill, uint64_t* stats, int grid,
                   hipStream_t st, const DevScene* scenes = nullptr, const RenderConsts* rcs = nullptr,
                   bool batch_env = false, bool batch_ext = false);
+// every bounce from `depth` (>= 1) on of the paths of state set `in`, in one
+// launch (k_shade, SH_TAIL); no traversal counts; with the radiance cache
+// `depth` lies beyond the query depth
+void launch_tail(const DevScene& sc, const DevPaths& P, int in, int out, uint32_t depth, const RenderConsts& rc,
+                 int matset, uint2* spill, uint64_t* stats, int grid, hipStream_t st,
+                 const DevScene* scenes = nullptr, const RenderConsts* rcs = nullptr, bool batch_env = false,
+                 bool batch_ext = false);
 int shade_material_set(uint32_t types_mask);
 // environment importance-sampling tables of a W x H float4 map; scratch
 // holds 1 + H 64-bit words

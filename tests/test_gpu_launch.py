@@ -106,3 +106,25 @@ def test_facade_launch_loop_equals_render(tmp_path, scene, cfg, W, H, frames):
     assert np.array_equal(acc_map[..., :3], acc.astype(np.float32))
     assert np.all(acc_map[..., 3] == frames)
     assert np.array_equal(disp_map, disp)
+
+
+# depths around the bounce where one launch takes over the rest of a batch
+# (1 or 3 at these sizes), a path count below one wave, and 2^18 + 1 paths
+@pytest.mark.parametrize("cfg,W,H,frames,depths", [
+    (ptamd.PT_SCENE_CORNELL, 7, 5, 1, (1, 2, 3)), (ptamd.PT_SCENE_CORNELL, 96, 64, 2, (1, 2, 16)),
+    (ptamd.PT_SCENE_RANDOM_SPHERES, 513, 511, 1, (1, 3, 4, 50)), (ptamd.PT_SCENE_MESHES, 61, 47, 3, (2, 12)),
+    (ptamd.PT_SCENE_NEXT_WEEK, 61, 47, 2, (2, 50)), (ptamd.PT_SCENE_MOVING_SPHERES, 61, 47, 2, (3, 50))])
+def test_last_bounces_in_one_launch_are_bit_identical(ctx, cfg, W, H, frames, depths):
+    sc = setup(ctx, cfg, W, H, 3 if cfg == ptamd.PT_SCENE_MESHES else 0)
+    flags = sc.info.flags | ptamd.PT_FLAG_KEEP_PATHS
+    for depth in depths:
+        say(f"[gpu] one launch for the last bounces: scene {cfg} {W}x{H} depth {depth}")
+        got = []
+        for extra in (0, ptamd.PT_FLAG_DIRECT):
+            p = sc.render_params(flags=flags | extra)
+            p.max_depth = depth
+            acc, st = image(ctx, p, 0, frames)
+            got.append((acc, *ctx.read_paths(W, H),
+                        np.array([st.extension_rays, st.shadow_rays, st.exhausted_paths, st.nan_paths])))
+        for a, b in zip(*got):
+            assert np.array_equal(a, b, equal_nan=True)
