@@ -470,15 +470,14 @@ PTD uint32_t collapse_expand(const BinTree& t, uint32_t m, int leaf_max, uint32_
 // next_base + o in slot order and appended to the next frontier
 PTD void collapse_emit(const BinTree& t, const uint32_t s[4], uint32_t o, int leaf_max, uint32_t next_base,
                        uint4* nd, uint32_t* next_frontier, uint32_t cap) {
-  uint32_t wl[6][4], ch[4], cn[4];
+  uint32_t wl[6][4], ref[4];
   for (int k = 0; k < 4; k++) {
     uint32_t r = s[k];
     if (r == EMPTY_CHILD) {
       wl[0][k] = __float_as_uint(FINF); wl[1][k] = __float_as_uint(-FINF);
       wl[2][k] = __float_as_uint(FINF); wl[3][k] = __float_as_uint(-FINF);
       wl[4][k] = __float_as_uint(FINF); wl[5][k] = __float_as_uint(-FINF);
-      ch[k] = EMPTY_CHILD;
-      cn[k] = 0;
+      ref[k] = EMPTY_REF;
       continue;
     }
     float4 lo, hi;
@@ -488,18 +487,16 @@ PTD void collapse_emit(const BinTree& t, const uint32_t s[4], uint32_t o, int le
     wl[4][k] = __float_as_uint(lo.z); wl[5][k] = __float_as_uint(hi.z);
     uint32_t sz = ref_size(t, r);
     if ((r & LEAF_BIT) || sz <= (uint32_t)leaf_max) {
-      ch[k] = ref_first(t, r);
-      cn[k] = sz;
+      ref[k] = LEAF_BIT | (sz << 28) | ref_first(t, r);
     } else {
-      ch[k] = next_base + o;
-      cn[k] = 0;
+      ref[k] = next_base + o;
       if (o < cap) next_frontier[o] = r;
       o++;
     }
   }
   for (int q = 0; q < 6; q++) nd[q] = make_uint4(wl[q][0], wl[q][1], wl[q][2], wl[q][3]);
-  nd[6] = make_uint4(ch[0], ch[1], ch[2], ch[3]);
-  nd[7] = make_uint4(cn[0], cn[1], cn[2], cn[3]);
+  nd[6] = make_uint4(ref[0], ref[1], ref[2], ref[3]);
+  nd[7] = make_uint4(0u, 0u, 0u, 0u);
 }
 
 // Breadth-first collapse of the binary hierarchy into BVH4 nodes: expand
@@ -618,8 +615,8 @@ __global__ void k_single_leaf(const float4* lo_box, const float4* hi_box, uint32
   nodes[3] = make_uint4(__float_as_uint(hi.y), e_hi.y, e_hi.z, e_hi.w);
   nodes[4] = make_uint4(__float_as_uint(lo.z), e_lo.y, e_lo.z, e_lo.w);
   nodes[5] = make_uint4(__float_as_uint(hi.z), e_hi.y, e_hi.z, e_hi.w);
-  nodes[6] = make_uint4(0u, EMPTY_CHILD, EMPTY_CHILD, EMPTY_CHILD);
-  nodes[7] = make_uint4(n, 0u, 0u, 0u);
+  nodes[6] = make_uint4(LEAF_BIT | (n << 28), EMPTY_REF, EMPTY_REF, EMPTY_REF);
+  nodes[7] = make_uint4(0u, 0u, 0u, 0u);
   root[0] = lo;
   root[1] = hi;
 }

@@ -970,6 +970,7 @@ pt_status pt_build_accel(pt_context* c, pt_accel_stats* out) {
   c->tlas_nodes = tn;
   c->total_prims_sorted = total_sorted;
   s.nodes = c->nodes_dev;
+  s.wide = c->total_nodes >= (1ull << 32) / 128 ? 1u : 0u;
   s.tlas_root = (uint32_t)blas_nodes;
   {
     // scene box = union of the top-level root's children
@@ -977,7 +978,7 @@ pt_status pt_build_accel(pt_context* c, pt_accel_stats* out) {
     HIPCHK(c, hipMemcpy(w, c->nodes_dev + 8ull * blas_nodes, 128, hipMemcpyDeviceToHost));
     float lo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, hi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
     for (int k = 0; k < 4; k++) {
-      if (w[24 + k] == EMPTY_CHILD) continue;
+      if (w[24 + k] == EMPTY_REF) continue;
       for (int a = 0; a < 3; a++) {
         float l, h;
         std::memcpy(&l, &w[8 * a + k], 4);
@@ -1027,7 +1028,18 @@ pt_status pt_read_accel(pt_context* c, uint32_t* nodes, uint64_t* num_nodes, uin
   if (num_nodes) *num_nodes = c->total_nodes;
   if (num_prims) *num_prims = c->total_prims_sorted;
   if (num_blas) *num_blas = (uint32_t)c->blas.size();
-  if (nodes) HIPCHK(c, hipMemcpy(nodes, c->nodes_dev, c->total_nodes * 128, hipMemcpyDeviceToHost));
+  if (nodes) {
+    HIPCHK(c, hipMemcpy(nodes, c->nodes_dev, c->total_nodes * 128, hipMemcpyDeviceToHost));
+    // the traversal's references as child and count words
+    for (uint64_t i = 0; i < c->total_nodes; i++) {
+      uint32_t* w = nodes + i * NODE_WORDS;
+      for (int k = 0; k < 4; k++) {
+        const uint32_t r = w[24 + k], n = (r & LEAF_BIT) ? (r >> 28) & 7u : 0u;
+        w[24 + k] = r == EMPTY_REF ? EMPTY_CHILD : (r & LEAF_BIT) ? (r & 0x0FFFFFFFu) : r;
+        w[28 + k] = n;
+      }
+    }
+  }
   if (prim_order) HIPCHK(c, hipMemcpy(prim_order, c->order_dev, c->total_prims_sorted * 4, hipMemcpyDeviceToHost));
   if (morton) HIPCHK(c, hipMemcpy(morton, c->morton_dev, c->total_prims_sorted * 4, hipMemcpyDeviceToHost));
   if (blas_info) {
@@ -1246,7 +1258,7 @@ pt_status pt_render(pt_context* c, const pt_render_params* rp, uint32_t frame_be
       if (rc.cache.query_depth < rp->max_depth) tail = std::max(tail, rc.cache.query_depth + 1);
       if (sort) tail = 0xFFFFFFFFu;
     }
-    if (count_trav || (rp->flags & PT_FLAG_DIRECT)) tail = 0xFFFFFFFFu;
+    if (count_trav || c->dsc.wide || (rp->flags & PT_FLAG_DIRECT)) tail = 0xFFFFFFFFu;
     for (uint32_t depth = 0; depth < rp->max_depth; depth++) {
       if (depth == tail) {
         hipEvent_t a = events ? mark() : nullptr;
@@ -1427,12 +1439,14 @@ pt_status pt_render(pt_context* c, const pt_render_params* rp, uint32_t frame_be
     out->paths = (uint64_t)frame_count * WH;
     out->extension_rays = st[STAT_EXT];
     out->shadow_rays = st[STAT_SHADOW];
-    out->node_fetches = st[STAT_NODES];
-    out->prim_fetches = st[STAT_PRIMS];
-    out->instance_fetches = st[STAT_INSTS];
-    out->shadow_node_fetches = st[STAT_SH_NODES];
-    out->shadow_prim_fetches = st[STAT_SH_PRIMS];
-    out->shadow_instance_fetches = st[STAT_SH_INSTS];
+    if (count_trav) {  // (wide scenes always count)
+      out->node_fetches = st[STAT_NODES];
+      out->prim_fetches = st[STAT_PRIMS];
+      out->instance_fetches = st[STAT_INSTS];
+      out->shadow_node_fetches = st[STAT_SH_NODES];
+      out->shadow_prim_fetches = st[STAT_SH_PRIMS];
+      out->shadow_instance_fetches = st[STAT_SH_INSTS];
+    }
     out->exhausted_paths = st[STAT_EXHAUSTED];
     out->nan_paths = st[STAT_NAN];
     out->cache_queries = c->cache_last_query;

@@ -177,14 +177,13 @@ PTD float isect_sphere(float4 s, v3 o, v3 d, float tmin) {
   return (-b + sq) / a;
 }
 // aarect.cu:20-69 (inclusive bounds); A = (a0, a1, b0, b1), k, axis.  The
-// plane distance multiplies by the ray's reciprocal direction `inv`
-// (1 / d per component, computed once per instance) where the reference
-// divides: one multiply instead of an IEEE division per test.
-PTD float isect_rect(float4 A, float k, int axis, v3 o, v3 d, v3 inv) {
+// plane distance multiplies by `inv`, the IEEE reciprocal of the ray
+// direction's `axis` component, where the reference divides.
+PTD float isect_rect(float4 A, float k, int axis, v3 o, v3 d, float inv) {
   float t, a, b;
-  if (axis == 0) { t = (k - o.x) * inv.x; a = o.y + t * d.y; b = o.z + t * d.z; }
-  else if (axis == 1) { t = (k - o.y) * inv.y; a = o.x + t * d.x; b = o.z + t * d.z; }
-  else { t = (k - o.z) * inv.z; a = o.x + t * d.x; b = o.y + t * d.y; }
+  if (axis == 0) { t = (k - o.x) * inv; a = o.y + t * d.y; b = o.z + t * d.z; }
+  else if (axis == 1) { t = (k - o.y) * inv; a = o.x + t * d.x; b = o.z + t * d.z; }
+  else { t = (k - o.z) * inv; a = o.x + t * d.x; b = o.y + t * d.y; }
   if (a < A.x || a > A.y || b < A.z || b > A.w) return FINF;
   return t;
 }
@@ -299,10 +298,19 @@ PTD v3 moving_center(float4 A, float4 B, float4 C, float time) {
 }
 
 // Watertight ray/triangle test (Woop, Benthin, Wald, JCGT 2(1), 2013).
+// The paper swaps kx and ky for a negative dominant component, to keep the
+// winding; here the axes stay cyclic.  The swap negates U, V and W (products
+// and differences round alike either way), hence det and T, and leaves t =
+// T / det and the barycentrics the same bits; the test accepts both signs.
 struct TriRay {
-  int kx, ky, kz;
+  int kz;
   float Sx, Sy, Sz;
 };
+// (x, y, z) -> components kx = kz + 1, ky = kz + 2 (mod 3), kz
+PTD v3 cyclic(v3 a, int kz) {
+  return mk3(kz == 0 ? a.y : (kz == 1 ? a.z : a.x), kz == 0 ? a.z : (kz == 1 ? a.x : a.y),
+             kz == 0 ? a.x : (kz == 1 ? a.y : a.z));
+}
 // a * b = hi + lo exactly (Dekker's product over Veltkamp's 12-bit split; no
 // fused multiply-add)
 PTD void two_prod(float a, float b, float& hi, float& lo) {
@@ -327,22 +335,20 @@ PTD TriRay tri_setup(v3 d) {
   TriRay r;
   float ax = fabsf(d.x), ay = fabsf(d.y), az = fabsf(d.z);
   r.kz = (ax > ay) ? (ax > az ? 0 : 2) : (ay > az ? 1 : 2);
-  r.kx = r.kz + 1 == 3 ? 0 : r.kz + 1;
-  r.ky = r.kx + 1 == 3 ? 0 : r.kx + 1;
-  if (comp(d, r.kz) < 0.0f) { int t = r.kx; r.kx = r.ky; r.ky = t; }
-  r.Sx = comp(d, r.kx) / comp(d, r.kz);
-  r.Sy = comp(d, r.ky) / comp(d, r.kz);
-  r.Sz = 1.0f / comp(d, r.kz);
+  const v3 c = cyclic(d, r.kz);
+  r.Sx = c.x / c.z;
+  r.Sy = c.y / c.z;
+  r.Sz = 1.0f / c.z;
   return r;
 }
 PTD bool tri_test(const TriRay& r, v3 o, v3 v0, v3 v1, v3 v2, float& t, float& b1, float& b2) {
-  v3 A = v0 - o, B = v1 - o, C = v2 - o;
-  float Ax = comp(A, r.kx) - r.Sx * comp(A, r.kz);
-  float Ay = comp(A, r.ky) - r.Sy * comp(A, r.kz);
-  float Bx = comp(B, r.kx) - r.Sx * comp(B, r.kz);
-  float By = comp(B, r.ky) - r.Sy * comp(B, r.kz);
-  float Cx = comp(C, r.kx) - r.Sx * comp(C, r.kz);
-  float Cy = comp(C, r.ky) - r.Sy * comp(C, r.kz);
+  const v3 A = cyclic(v0 - o, r.kz), B = cyclic(v1 - o, r.kz), C = cyclic(v2 - o, r.kz);
+  float Ax = A.x - r.Sx * A.z;
+  float Ay = A.y - r.Sy * A.z;
+  float Bx = B.x - r.Sx * B.z;
+  float By = B.y - r.Sy * B.z;
+  float Cx = C.x - r.Sx * C.z;
+  float Cy = C.y - r.Sy * C.z;
   float U = Cx * By - Cy * Bx;
   float V = Ax * Cy - Ay * Cx;
   float W = Bx * Ay - By * Ax;
@@ -354,9 +360,9 @@ PTD bool tri_test(const TriRay& r, v3 o, v3 v0, v3 v1, v3 v2, float& t, float& b
   if ((U < 0.0f || V < 0.0f || W < 0.0f) && (U > 0.0f || V > 0.0f || W > 0.0f)) return false;
   float det = U + V + W;
   if (det == 0.0f) return false;
-  float Az = r.Sz * comp(A, r.kz);
-  float Bz = r.Sz * comp(B, r.kz);
-  float Cz = r.Sz * comp(C, r.kz);
+  float Az = r.Sz * A.z;
+  float Bz = r.Sz * B.z;
+  float Cz = r.Sz * C.z;
   float T = U * Az + V * Bz + W * Cz;
   float rcp = 1.0f / det;
   t = T * rcp;

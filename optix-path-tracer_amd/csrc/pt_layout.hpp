@@ -13,15 +13,19 @@ namespace pt {
 //   words  0.. 3  lo.x[4]     words  4.. 7  hi.x[4]
 //   words  8..11  lo.y[4]     words 12..15  hi.y[4]
 //   words 16..19  lo.z[4]     words 20..23  hi.z[4]
-//   words 24..27  child[4]: internal -> node index within its structure,
-//                 leaf -> first sorted primitive, empty -> 0xFFFFFFFF
-//   words 28..31  count[4]: 0 internal / empty, else leaf primitive count
+//   words 24..27  ref[4]: the traversal's references, see below
+//   words 28..31  unused (pt_read_accel returns child[4] in words 24..27 and
+//                 the leaf counts here)
+// An empty slot's planes are lo = +inf, hi = -inf.
 constexpr int NODE_WORDS = 32;
 constexpr int BLAS_LEAF_MAX = 4;
 constexpr int TLAS_LEAF_MAX = 1;
-// Traversal stack references: internal node index, or
-// LEAF_BIT | (count - 1) << 28 | first.
+// Traversal references, in the nodes and on the stack: the index of an
+// internal node within its structure, or LEAF_BIT | count << 28 | first
+// sorted primitive of a leaf; an empty slot is a leaf of no primitives.
 constexpr uint32_t LEAF_BIT = 1u << 31;
+constexpr uint32_t EMPTY_REF = LEAF_BIT;
+// no child yet (build)
 constexpr uint32_t EMPTY_CHILD = 0xFFFFFFFFu;
 
 // ------------------------------------------------------------ records
@@ -40,16 +44,17 @@ constexpr int INST_WORDS = 32;
 // lane in LDS, STK_SPILL more per thread in HBM.
 constexpr int BLOCK = 256;
 constexpr int STK_LDS = 16;
+constexpr int STK_LDS_SHADE = 12;  // shading kernel (shadow rays)
 // every thread owns STK_TOTAL entries in all: the ones beyond its kernel's
 // LDS entries spill to its HBM slice of STK_TOTAL entries
 constexpr int STK_TOTAL = 64;
 constexpr int STK_SPILL = STK_TOTAL - STK_LDS;
 // buckets per guide table of the environment sampler's searches
 constexpr uint32_t ENV_GUIDE = 64;
-// closest-hit kernel (k_extend) in scenes with meshes and in the camera-ray
-// pass: LDS entries per lane and occupancy target (waves per SIMD); 16
-// entries x 8 B x 256 lanes is 32 KB per block, which with up to 96 VGPRs
-// holds 5 waves per SIMD (the other instantiations: extend_waves)
+// closest-hit kernel (k_extend): LDS entries per lane in scenes with meshes,
+// and the occupancy target (waves per SIMD) of the bounce rays of one scene;
+// 16 entries x 8 B x 256 lanes is 32 KB per block, which with up to 96 VGPRs
+// holds 5 waves per SIMD
 #ifndef PT_EXTEND_STK
 #define PT_EXTEND_STK 16
 #endif
@@ -115,6 +120,7 @@ struct DevMesh {
 // Everything a kernel needs to see of the scene, passed by value.
 struct DevScene {
   const uint4* nodes;  // all BVH4 nodes (every BLAS, then the TLAS)
+  uint32_t wide;       // the nodes take 4 GB or more: 64-bit offsets
   uint32_t tlas_root;  // absolute node index of the TLAS root
   uint32_t num_instances;
   const uint4* insts;  // instance records in top-level order

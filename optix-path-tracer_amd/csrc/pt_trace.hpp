@@ -15,15 +15,13 @@ namespace pt {
 
 template <int NL>
 struct StackT {
-  uint32_t* ref;  // LDS column, stride BLOCK
-  float* tn;
-  uint2* spill;   // this thread's HBM slice (STK_TOTAL entries)
+  uint2* lds;    // LDS column (reference, entry distance), stride BLOCK
+  uint2* spill;  // this thread's HBM slice (STK_TOTAL entries)
   int sp;
   uint32_t* overflow;
   PTD void put(int pos, uint32_t r, float t) {
     if (pos < NL) {
-      ref[pos * BLOCK] = r;
-      tn[pos * BLOCK] = t;
+      lds[pos * BLOCK] = make_uint2(r, __float_as_uint(t));
     } else if (pos < STK_TOTAL) {
       spill[pos - NL] = make_uint2(r, __float_as_uint(t));
     } else {
@@ -32,17 +30,17 @@ struct StackT {
   }
   PTD void pop(uint32_t& r, float& t) {
     sp--;
-    if (sp < NL) {
-      r = ref[sp * BLOCK];
-      t = tn[sp * BLOCK];
-    } else if (sp < STK_TOTAL) {
-      uint2 e = spill[sp - NL];
-      r = e.x;
-      t = __uint_as_float(e.y);
-    } else {
-      r = EMPTY_CHILD;
-      t = FINF;
-    }
+    uint2 e = make_uint2(EMPTY_REF, __float_as_uint(FINF));
+    if (sp < NL) e = lds[sp * BLOCK];
+    else if (sp < STK_TOTAL) e = spill[sp - NL];
+    r = e.x;
+    t = __uint_as_float(e.y);
+  }
+  // three entries fit the LDS part in every lane
+  PTD bool room() const { return __ballot(sp > NL - 3) == 0; }
+  PTD void push_lds(uint32_t r, float t) {
+    lds[sp * BLOCK] = make_uint2(r, __float_as_uint(t));
+    sp++;
   }
 };
 using Stack = StackT<STK_LDS>;
@@ -53,9 +51,11 @@ PTD float4 as_f4(uint4 u) {
 
 struct HitOut {
   float t;
-  int inst, prim;  // original instance id and primitive index (-1: miss)
-  int pos;         // instance position in top-level order
+  int prim;  // original primitive index (-1: miss)
+  int pos;   // instance position in top-level order (-1: miss)
 };
+// original instance id of the instance at top-level position pos
+PTD int inst_at(const DevScene& sc, int pos) { return (int)sc.insts[(size_t)pos * 8 + 3].w; }
 
 struct TraceCounts {
   uint32_t nodes, prims, insts;
@@ -80,6 +80,7 @@ PTD float slab_test(float lox, float hix, float loy, float hiy, float loz, float
 // boxes, meshes) may occur; the tests of the other kinds (and the
 // triangle test's per-instance ray setup) are compiled out.
 constexpr int KIND_ALL = 15;
+constexpr uint32_t TRIPS_MAX = 1u << 22;
 // The traversal of one ray as a resumable state: begin() sets it up, each
 // step() does one trip of the loop (a pop, one internal node, one leaf's
 // primitives or an instance entry) and returns false once the ray is done
@@ -93,42 +94,58 @@ constexpr int KIND_ALL = 15;
 // kernels carry no trace of the early exit (a runtime-false flag still
 // changes their traversal loop's code and costs them about a tenth of
 // their time).
-template <bool COUNT, bool EXT = false, int KINDS = KIND_ALL, bool ANY = false>
+template <bool COUNT, bool EXT = false, int KINDS = KIND_ALL, bool ANY = false, bool WIDE = false>
 struct Tracer {
   static constexpr bool SPH = (KINDS & 1) != 0, RECT = (KINDS & 2) != 0, BOX = (KINDS & 4) != 0,
                         MESH = (KINDS & 8) != 0;
+  // FAST (kernels that do not count): the node test of node_fast
+  static constexpr bool FAST = !COUNT;
+  // rect and box tests (and the exact slab test) take the IEEE reciprocal
+  // direction: kept per instance, or, next to meshes (no registers to spare),
+  // formed by each test
+  static constexpr bool KEEP_INV = COUNT || ((RECT || BOX) && !MESH);
   HitOut h;
-  v3 o, d, winv, ro, rd, rinv;
+  v3 o, d, ro, rd, rinv;
+  // FAST: bounded reciprocal direction; -o * inv moved outward for near and
+  // far planes; byte offsets of the near planes in a node
+  v3 finv, nb, fb;
+  uint32_t sx, sy, sz;
   float tmin, time;
   uint32_t vseed;
   TriRay tr;
   int cur;      // instance slot in top-level order, -1 = top level
   int base_sp;  // stack depth when the instance was entered
-  uint32_t node_base, prim_base, kind, inst_id;
+  uint32_t node_base, prim_base, kind;
+  bool moved;   // the instance in hand has a transform: ro, rd are its own
   // the entry in hand: the top-level root first; the nearest child of each
   // node and an instance's root are taken directly instead of through the
   // stack, which visits the same nodes in the same order
   uint32_t ref;
-  float etn;
   bool have, any_hit;
-  // bound on loop trips: a well-formed structure never comes close
-  uint32_t trips;
+
+  // a candidate of the instance in hand as far as the hit: the smaller
+  // (instance, primitive) wins
+  PTD bool wins_tie(const DevScene& sc, int orig) const {
+    const int a = inst_at(sc, cur), b = inst_at(sc, h.pos);
+    return a < b || (a == b && orig < h.prim);
+  }
+  PTD v3 exact_inv() const {
+    return KEEP_INV ? rinv : mk3(1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z);
+  }
 
   // the watertight test of one triangle record and, when it is nearer (or
   // as near with the smaller key), its acceptance; true when an any-hit
   // query ends here
-  PTD bool offer_tri(float4 a, float4 b, float4 c, TraceCounts& cnt) {
+  PTD bool offer_tri(const DevScene& sc, float4 a, float4 b, float4 c, TraceCounts& cnt) {
     if (COUNT) cnt.prims++;
     float t = FINF, b1, b2;
     if (!tri_test(tr, ro, mk3(a), mk3(b), mk3(c), t, b1, b2)) t = FINF;
     const uint32_t orig = __float_as_uint(a.w);
     if (!(t > tmin)) return false;
     bool take = t < h.t;
-    if (!take && t == h.t && h.inst >= 0)
-      take = ((int)inst_id < h.inst) || ((int)inst_id == h.inst && (int)orig < h.prim);
+    if (!take && t == h.t && h.pos >= 0) take = wins_tie(sc, (int)orig);
     if (!take) return false;
     h.t = t;
-    h.inst = (int)inst_id;
     h.prim = (int)orig;
     h.pos = cur;
     return ANY && any_hit;
@@ -137,49 +154,156 @@ struct Tracer {
   template <class ST>
   PTD void begin(const DevScene& sc, v3 o_, v3 d_, float tmin_, float tmax, ST& st, uint32_t vseed_ = 0u,
                  float time_ = 0.f, bool any_hit_ = false) {
-    h = HitOut{tmax, -1, -1, -1};
+    h = HitOut{tmax, -1, -1};
     o = o_;
     d = d_;
     tmin = tmin_;
     time = time_;
     vseed = vseed_;
     any_hit = any_hit_;
-    winv = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
     ro = o;
     rd = d;
-    rinv = winv;
-    tr = TriRay{0, 1, 2, 0.f, 0.f, 0.f};
+    setup();
+    moved = false;
+    tr = TriRay{0, 0.f, 0.f, 0.f};
     cur = -1;
     base_sp = 0;
     node_base = sc.tlas_root;
     prim_base = 0;
     kind = 0;
-    inst_id = 0;
     st.sp = 0;
     ref = 0u;
-    etn = tmin;
     have = true;
-    trips = 0;
+  }
+
+  // Constants of node_fast for the ray (ro, rd): the reciprocal of each
+  // component, at most 2^100 in magnitude (a zero component gives no inf - inf
+  // with the scene's planes), and the two offsets.  A component that is NaN,
+  // infinite or above 2^100 gives NaN distances, which the minima and maxima
+  // pass over: that axis then rejects nothing.
+  PTD static float bound_rcp(float x) {
+    float m = fabsf(__builtin_amdgcn_rcpf(x));
+    m = m > 0x1p100f ? 0x1p100f : m;
+    m = m < 0x1p-100f ? __builtin_nanf("") : m;
+    return copysignf(m, x);
+  }
+  PTD void setup() {
+    if (KEEP_INV) rinv = mk3(1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z);
+    if (FAST) fast_setup();
+  }
+  PTD void fast_setup() {
+    finv = mk3(bound_rcp(rd.x), bound_rcp(rd.y), bound_rcp(rd.z));
+    const v3 a = mk3(ro.x * finv.x, ro.y * finv.y, ro.z * finv.z);
+    const v3 e = mk3(fabsf(a.x) * 0x1p-21f, fabsf(a.y) * 0x1p-21f, fabsf(a.z) * 0x1p-21f);
+    nb = mk3(-a.x - e.x, -a.y - e.y, -a.z - e.z);
+    fb = mk3(e.x - a.x, e.y - a.y, e.z - a.z);
+    sx = finv.x < 0.f ? 16u : 0u;
+    sy = finv.y < 0.f ? 48u : 32u;
+    sz = finv.z < 0.f ? 80u : 64u;
+  }
+
+  // One internal node: the children the ray may enter, the nearest taken
+  // next and the others on the stack, second nearest on top.
+  //
+  // A plane's distance is one fused multiply-add, plane * inv + (-o * inv),
+  // the planes a component meets first (near) and last (far) picked by their
+  // address; the exact test (slab_test) subtracts, multiplies and sorts the
+  // two distances.  Rounding: with u = 2^-24, the reciprocal is off by 2 u,
+  // o * inv by u, the offset's sum and the fma by u each, so a distance is
+  // off by less than 6 u (|o inv| + |plane inv - o inv|).  The offsets move
+  // every plane outward by 8 u |o inv| and the far distance grows by 32 u of
+  // itself, which also covers the exact test's own rounding: the children
+  // taken are those of the exact test, and now and then one more, whose
+  // primitives cannot win a closer hit.  Empty slots (inf planes) always
+  // fail, or, for a ray of NaNs, lead to a leaf of no primitives.
+  //
+  // Sorted by a network of five exchanges, reference and distance stored
+  // together, a node takes about 180 instructions where the exact test with
+  // its ranking by pairwise comparisons takes 450.  4 M random rays in the
+  // mesh scene 1.18 -> 0.96 ms, one 1080p frame of it 4.57 -> 4.0 ms, its
+  // camera-ray launch at 96 spp 16.7 -> 15.6 ms and the next bounce 13.3 ->
+  // 11.5 ms; the Cornell box, whose rays meet 2.3 nodes, is unchanged.
+  PTD void exchange(float& ta, uint32_t& ra, float& tb, uint32_t& rb) {
+    const bool s = tb < ta;
+    const float t0 = s ? tb : ta, t1 = s ? ta : tb;
+    const uint32_t r0 = s ? rb : ra, r1 = s ? ra : rb;
+    ta = t0; tb = t1; ra = r0; rb = r1;
+  }
+  template <class ST>
+  PTD void node_fast(const DevScene& sc, ST& st) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    f4 nx, ny, nz, fx, fy, fz;
+    u4 cr;
+    const uint32_t index = node_base + ref;
+    if constexpr (WIDE) {
+      typedef const __attribute__((address_space(1))) char* gp;
+      const uint64_t p = (uint64_t)(gp)sc.nodes + ((uint64_t)index << 7);
+      auto ld = [&](uint32_t k) { return *(const __attribute__((address_space(1))) f4*)(p | k); };
+      nx = ld(sx); fx = ld(sx ^ 16u);
+      ny = ld(sy); fy = ld(sy ^ 16u);
+      nz = ld(sz); fz = ld(sz ^ 16u);
+      cr = *(const __attribute__((address_space(1))) u4*)(p + 96u);
+    } else {
+      const char* b = reinterpret_cast<const char*>(sc.nodes);
+      const uint32_t p = index << 7;
+      auto ld = [&](uint32_t k) { return *reinterpret_cast<const f4*>(b + (p | k)); };
+      nx = ld(sx); fx = ld(sx ^ 16u);
+      ny = ld(sy); fy = ld(sy ^ 16u);
+      nz = ld(sz); fz = ld(sz ^ 16u);
+      cr = *reinterpret_cast<const u4*>(b + (p | 96u));
+    }
+    auto slab = [&](float ax, float bx, float ay, float by, float az, float bz) {
+      const float tn = fmaxf(fmaxf(fmaxf(__builtin_fmaf(ax, finv.x, nb.x), __builtin_fmaf(ay, finv.y, nb.y)),
+                                   __builtin_fmaf(az, finv.z, nb.z)), tmin);
+      float tf = fminf(fminf(fminf(__builtin_fmaf(bx, finv.x, fb.x), __builtin_fmaf(by, finv.y, fb.y)),
+                             __builtin_fmaf(bz, finv.z, fb.z)), h.t);
+      tf = __builtin_fmaf(fabsf(tf), 0x1p-19f, tf);
+      return tn <= tf ? tn : FINF;
+    };
+    float t0 = slab(nx.x, fx.x, ny.x, fy.x, nz.x, fz.x), t1 = slab(nx.y, fx.y, ny.y, fy.y, nz.y, fz.y);
+    float t2 = slab(nx.z, fx.z, ny.z, fy.z, nz.z, fz.z), t3 = slab(nx.w, fx.w, ny.w, fy.w, nz.w, fz.w);
+    uint32_t r0 = cr.x, r1 = cr.y, r2 = cr.z, r3 = cr.w;
+    exchange(t0, r0, t1, r1);
+    exchange(t2, r2, t3, r3);
+    exchange(t0, r0, t2, r2);
+    exchange(t1, r1, t3, r3);
+    exchange(t1, r1, t2, r2);
+    ref = r0;
+    have = t0 < FINF;
+    if (st.room()) {
+      if (t3 < FINF) st.push_lds(r3, t3);
+      if (t2 < FINF) st.push_lds(r2, t2);
+      if (t1 < FINF) st.push_lds(r1, t1);
+    } else {
+      if (t3 < FINF) { st.put(st.sp, r3, t3); st.sp++; }
+      if (t2 < FINF) { st.put(st.sp, r2, t2); st.sp++; }
+      if (t1 < FINF) { st.put(st.sp, r1, t1); st.sp++; }
+    }
   }
 
   template <class ST>
   PTD bool step(const DevScene& sc, ST& st, TraceCounts& cnt) {
-    if (!(++trips < (1u << 22))) return false;
     if (!have) {
       if (cur >= 0 && st.sp == base_sp) {
         cur = -1;
         node_base = sc.tlas_root;
-        ro = o; rd = d; rinv = winv;
+        if (moved) {
+          ro = o; rd = d;
+          setup();
+        }
       }
       if (st.sp == 0) return false;
+      float etn;
       st.pop(ref, etn);
-      if (ref == EMPTY_CHILD || etn > h.t) return true;
+      if (etn > h.t) return true;
     }
     have = false;
     if (ref & LEAF_BIT) {
       uint32_t first = ref & 0x0FFFFFFFu;
-      uint32_t count = ((ref >> 28) & 7u) + 1u;
+      uint32_t count = (ref >> 28) & 7u;
       if (cur < 0) {
+        if (FAST && count == 0) return true;  // an empty slot (a ray of NaNs)
         // enter the instance at top-level position `first`
         const uint4* ir = sc.insts + (size_t)first * 8;
         float4 w0 = as_f4(ir[0]);
@@ -190,7 +314,6 @@ struct Tracer {
         node_base = info.x;
         prim_base = info.y;
         kind = info.z & 0xFFu;
-        inst_id = info.w;
         // the object-space ray is formed for every instance and kept where
         // the instance has a transform: formed behind a branch on that flag,
         // the matrix would be loaded only after the flag arrives (a second
@@ -201,7 +324,8 @@ struct Tracer {
         const v3 xo = xf_point(w0, w1, w2, o), xd = xf_vector(w0, w1, w2, d);
         ro = mk3(xf ? xo.x : o.x, xf ? xo.y : o.y, xf ? xo.z : o.z);
         rd = mk3(xf ? xd.x : d.x, xf ? xd.y : d.y, xf ? xd.z : d.z);
-        if (xf) rinv = mk3(1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z);
+        moved = xf;
+        if (xf) setup();
         if (MESH && kind == PT_GEOM_MESH) tr = tri_setup(rd);
         cur = (int)first;
         base_sp = st.sp;
@@ -219,8 +343,8 @@ struct Tracer {
           const uint32_t p1 = two ? p0 + 1 : p0;
           const float4 a0 = sc.tri[3 * p0], b0 = sc.tri[3 * p0 + 1], c0 = sc.tri[3 * p0 + 2];
           const float4 a1 = sc.tri[3 * p1], b1 = sc.tri[3 * p1 + 1], c1 = sc.tri[3 * p1 + 2];
-          if (offer_tri(a0, b0, c0, cnt)) return false;
-          if (two && offer_tri(a1, b1, c1, cnt)) return false;
+          if (offer_tri(sc, a0, b0, c0, cnt)) return false;
+          if (two && offer_tri(sc, a1, b1, c1, cnt)) return false;
         }
         return true;
       }
@@ -233,16 +357,21 @@ struct Tracer {
           t = isect_sphere(sc.sph[p], ro, rd, tmin);
         } else if (RECT && kind == PT_GEOM_RECTS) {
           float4 A = sc.rect[2 * p], B = sc.rect[2 * p + 1];
-          t = isect_rect(A, B.x, (int)__float_as_uint(B.y), ro, rd, rinv);
+          const int axis = (int)__float_as_uint(B.y);
+          if (KEEP_INV) {
+            t = isect_rect(A, B.x, axis, ro, rd, axis == 0 ? rinv.x : (axis == 1 ? rinv.y : rinv.z));
+          } else {
+            t = isect_rect(A, B.x, axis, ro, rd, 1.0f / (axis == 0 ? rd.x : (axis == 1 ? rd.y : rd.z)));
+          }
           orig = __float_as_uint(B.w);
         } else if (BOX && kind == PT_GEOM_BOXES) {
           float4 lo = sc.box[2 * p], hi = sc.box[2 * p + 1];
-          t = isect_box(mk3(lo), mk3(hi), ro, rinv, tmin);
+          t = isect_box(mk3(lo), mk3(hi), ro, exact_inv(), tmin);
           orig = __float_as_uint(lo.w);
         } else if (EXT && kind == PT_GEOM_VOLUMES) {
           float4 A = sc.vol[2 * p], B = sc.vol[2 * p + 1];
           orig = __float_as_uint(B.w) & 0x7FFFFFFFu;
-          t = isect_volume(A, B, ro, rd, tmin, vol_xi(vseed, orig, inst_id));
+          t = isect_volume(A, B, ro, rd, tmin, vol_xi(vseed, orig, (uint32_t)inst_at(sc, cur)));
         } else if (EXT && kind == PT_GEOM_CYLINDERS) {
           float4 A = sc.cyl[2 * p], B = sc.cyl[2 * p + 1];
           orig = __float_as_uint(B.w);
@@ -260,14 +389,13 @@ struct Tracer {
         }
         if (!(t > tmin)) continue;
         bool take = t < h.t;
-        if (!take && t == h.t && h.inst >= 0) {
+        if (!take && t == h.t && h.pos >= 0) {
           if (SPH && kind == PT_GEOM_SPHERES) orig = sc.sph_idx[p];
-          take = ((int)inst_id < h.inst) || ((int)inst_id == h.inst && (int)orig < h.prim);
+          take = wins_tie(sc, (int)orig);
         }
         if (take) {
           if (SPH && kind == PT_GEOM_SPHERES && orig == 0xFFFFFFFFu) orig = sc.sph_idx[p];
           h.t = t;
-          h.inst = (int)inst_id;
           h.prim = (int)orig;
           h.pos = cur;
           if (ANY && any_hit) return false;
@@ -276,15 +404,18 @@ struct Tracer {
       return true;
     }
     // internal node
+    if constexpr (FAST) {
+      node_fast(sc, st);
+      return true;
+    }
     if (COUNT) cnt.nodes++;
     const uint4* nd = sc.nodes + (size_t)(node_base + ref) * 8;
-    uint4 q0 = nd[0], q1 = nd[1], q2 = nd[2], q3 = nd[3], q4 = nd[4], q5 = nd[5], q6 = nd[6], q7 = nd[7];
+    uint4 q0 = nd[0], q1 = nd[1], q2 = nd[2], q3 = nd[3], q4 = nd[4], q5 = nd[5], q6 = nd[6];
     const uint32_t lox[4] = {q0.x, q0.y, q0.z, q0.w}, hix[4] = {q1.x, q1.y, q1.z, q1.w};
     const uint32_t loy[4] = {q2.x, q2.y, q2.z, q2.w}, hiy[4] = {q3.x, q3.y, q3.z, q3.w};
     const uint32_t loz[4] = {q4.x, q4.y, q4.z, q4.w}, hiz[4] = {q5.x, q5.y, q5.z, q5.w};
-    const uint32_t chd[4] = {q6.x, q6.y, q6.z, q6.w}, cnc[4] = {q7.x, q7.y, q7.z, q7.w};
+    const uint32_t cref[4] = {q6.x, q6.y, q6.z, q6.w};
     float tn[4];
-    uint32_t cref[4];
     // every slot's test runs and empty slots are masked afterwards: a test
     // behind a branch on the slot lets the compiler load that slot's planes
     // only after the child words arrive, a second memory round trip per node
@@ -293,8 +424,7 @@ struct Tracer {
       const float ts = slab_test(__uint_as_float(lox[c]), __uint_as_float(hix[c]), __uint_as_float(loy[c]),
                                  __uint_as_float(hiy[c]), __uint_as_float(loz[c]), __uint_as_float(hiz[c]), ro, rinv,
                                  tmin, h.t);
-      tn[c] = chd[c] != EMPTY_CHILD ? ts : FINF;
-      cref[c] = cnc[c] ? (LEAF_BIT | ((cnc[c] - 1u) << 28) | chd[c]) : chd[c];
+      tn[c] = cref[c] != EMPTY_REF ? ts : FINF;
     }
     // rank by (tn, slot): the nearest is taken next, the others go on the
     // stack with the second nearest on top
@@ -312,7 +442,6 @@ struct Tracer {
         // the cull a pop would apply (the slab test's far bound is 2^-22 loose)
         if (!(tn[c] > h.t)) {
           ref = cref[c];
-          etn = tn[c];
           have = true;
         }
       } else {
@@ -324,12 +453,13 @@ struct Tracer {
   }
 };
 
-template <bool COUNT, bool EXT = false, int KINDS = KIND_ALL, bool ANY = false, class ST>
+template <bool COUNT, bool EXT = false, int KINDS = KIND_ALL, bool ANY = false, bool WIDE = false, class ST>
 PTD HitOut trace_closest(const DevScene& sc, v3 o, v3 d, float tmin, float tmax, ST& st, TraceCounts& cnt,
                          uint32_t vseed = 0u, float time = 0.f, bool any_hit = false) {
-  Tracer<COUNT, EXT, KINDS, ANY> t;
+  Tracer<COUNT, EXT, KINDS, ANY, WIDE> t;
   t.begin(sc, o, d, tmin, tmax, st, vseed, time, any_hit);
-  while (t.step(sc, st, cnt)) {
+  // the bound (a well-formed structure never comes close) is wave-uniform
+  for (uint32_t trips = 0; trips < TRIPS_MAX && t.step(sc, st, cnt); trips++) {
   }
   return t.h;
 }

@@ -723,3 +723,69 @@ def test_vector_texture_paths_match_oracle(ctx):
     bad.instance(ptamd.PT_GEOM_SPHERES, 0, 1)
     with pytest.raises(ptamd.PtError):
         ctx.set_scene(bad.desc())
+
+
+def awkward_rays(n, lo, hi, seed):
+    """Random rays with the components that an interval test meets at its
+    edges: zeros, denormals, huge and tiny directions, axis-parallel rays,
+    origins on box planes and far away, bounded and empty intervals, and (a
+    few) infinities and NaNs."""
+    rng = np.random.default_rng(seed)
+    lo, hi = np.array(lo, np.float64), np.array(hi, np.float64)
+    org = rng.uniform(lo, hi, (n, 3))
+    d = rng.normal(size=(n, 3))
+    k = np.arange(n)
+    rows = k[k % 7 == 1]
+    d[rows, rng.integers(0, 3, len(rows))] = 0.0
+    rows = k[k % 7 == 2]
+    keep = rng.integers(0, 3, len(rows))
+    d[rows] = np.where(np.arange(3) == keep[:, None], d[rows], rng.choice([0.0, -0.0, 1e-42, -1e-30], (len(rows), 3)))
+    rows = k[k % 7 == 3]
+    d[rows] *= 10.0 ** rng.uniform(-18, 18, (len(rows), 1))
+    rows = k[k % 7 == 4]
+    org[rows] = np.round(org[rows])
+    rows = k[k % 7 == 5]
+    org[rows] = lo + (hi - lo) * rng.choice([-30.0, 0.0, 1.0, 40.0], (len(rows), 3))
+    d[rows] = rng.uniform(lo, hi, (len(rows), 3)) - org[rows]
+    rays = np.zeros(n, ptamd.RAY_DTYPE)
+    rays["org"], rays["dir"] = org, d
+    rays["tmin"] = rng.choice([0.0, 1e-6, 1e-3, 0.5, -1.0], n)
+    rays["tmax"] = np.where(rng.random(n) < 0.5, np.inf, rng.uniform(0, 2, n) * np.linalg.norm(hi - lo))
+    rows = k[k % 97 == 6]
+    bad = rng.choice([np.inf, -np.inf, np.nan], len(rows))
+    half = len(rows) // 2
+    rays["dir"][rows[:half], 0] = bad[:half]
+    rays["org"][rows[half:], 1] = bad[half:]
+    return rays
+
+
+# The kernels that count use the exact slab test, the others a conservative
+# one with fused multiply-adds: they visit the same leaves and at times one
+# more, so their hit is never behind the exact test's, or behind it in a tie.
+# Ordinary rays give the same hit bit for bit; a ray from 30 scene sizes away,
+# of length 1e18 or with a negative tmin may meet a primitive (a sphere whose
+# discriminant has lost its digits, an equal distance) whose box the exact
+# test's rounding misses.  Infinities and NaNs have no defined hit; they are
+# traced to an end.
+@pytest.mark.parametrize("cfg,variant,lo,hi", [
+    (ptamd.PT_SCENE_CORNELL, 0, (0, 0, 0), (555, 555, 555)), (ptamd.PT_SCENE_RANDOM_SPHERES, 0, (-11, 0, -11), (11, 2, 11)),
+    (ptamd.PT_SCENE_MESHES, 1, (-12, -8, -12), (12, 8, 12)), (ptamd.PT_SCENE_MESHES, 5, (-12, -8, -12), (12, 8, 12)),
+    (ptamd.PT_SCENE_NEXT_WEEK, 0, (-400, 0, -300), (600, 550, 600))])
+def test_fast_and_exact_node_tests_agree(ctx, cfg, variant, lo, hi):
+    sc = ptamd.Scene(cfg, 64, 64, variant)
+    ctx.set_scene(sc.desc)
+    ctx.build_accel()
+    for n in (1, 63, 200_003):
+        say(f"[gpu] node tests scene {cfg} variant {variant}: {n} rays")
+        rays = awkward_rays(n, lo, hi, n)
+        a = ctx.trace_closest(rays)
+        b, _ = ctx.trace_closest(rays, counted=True)
+        differ = (a["t"] != b["t"]) | (a["inst"] != b["inst"]) | (a["prim"] != b["prim"])
+        tie = (a["t"] == b["t"]) & ((a["inst"] < b["inst"]) | ((a["inst"] == b["inst"]) & (a["prim"] < b["prim"])))
+        k = np.arange(n)
+        finite = np.isfinite(rays["org"]).all(1) & np.isfinite(rays["dir"]).all(1)
+        assert np.all(~differ | (a["t"] < b["t"]) | tie | ~finite)
+        plain = (k % 7 != 3) & (k % 7 != 5) & finite & (rays["tmin"] >= 0)
+        assert not np.any(differ & plain)
+        assert differ.sum() <= 1e-4 * n
+    assert (a["inst"] >= 0).mean() > 0.1
