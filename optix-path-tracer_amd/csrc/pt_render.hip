@@ -61,8 +61,8 @@ __global__ __launch_bounds__(BLOCK) void k_trace_occluded(DevScene sc, const pt_
 }
 
 // ------------------------------------------------------ wavefront kernels
-// Slot of position p in a batch of nslots.  Slots come in 64-slot chunks
-// (64 consecutive pixels of one row, coherent camera rays); the chunk index
+// Slot index of position p in a batch of nslots.  Slots come in 64-slot chunks
+// (an 8 x 8 tile of pixels, coherent camera rays); the chunk index
 // goes through a keyed 4-round Feistel permutation, cycle-walked into the Q
 // full chunks, so that the chunks a wave owns come from all over the
 // batch's frames and every wave keeps about the image-average share of
@@ -89,20 +89,52 @@ PTD uint32_t slot_of(uint32_t p, uint32_t nslots) {
   return (x << 6) | (p & 63u);
 }
 
+// Pixel r of a frame in tile order: whole 8 x 8 tiles row by row, 64 pixels
+// each, then the columns right of them and the rows above.  A wave's 64 camera
+// rays start close together in both directions and meet fewer different nodes,
+// triangles and texels than along 64 pixels of one row: mesh still at 96 spp,
+// camera-ray launch 15.6 -> 12.1 ms and its shading 16.8 -> 14.9 ms.
+PTD void tile_pixel(uint32_t r, uint32_t W, uint32_t H, uint32_t& x, uint32_t& y) {
+  const uint32_t tw = W >> 3, th = H >> 3, whole = tw * th * 64u;
+  if (r < whole) {
+    const uint32_t t = r >> 6, ty = t / tw;
+    x = (t - ty * tw) * 8u + (r & 7u);
+    y = ty * 8u + ((r >> 3) & 7u);
+    return;
+  }
+  uint32_t q = r - whole;
+  const uint32_t cw = W & 7u, right = cw * th * 8u;
+  const bool in_right = q < right;
+  if (!in_right) q -= right;
+  const uint32_t w = in_right ? cw : W;
+  y = q / w;
+  x = q - y * w + (in_right ? tw * 8u : 0u);
+  y += in_right ? 0u : th * 8u;
+}
+
 // raygen.cu:148-168 renderPixel up to the first rtTrace, raygen.cu:50-64
 // generateRay, raygen.cu:66-74 color() set-up.
-// One camera path: slot s (frame `frame` of the scene, pixel `pix`) at
-// position p of state set 0; in a batch of scenes the RNG state's top byte
+// One camera path: slot s0 + launch index of pixel r of frame `frame` of the
+// scene, at position p of state set 0; in a batch of scenes the RNG state's top byte
 // is replaced by the scene index.  Returns the stored ray and its time.
 struct PathStart {
   float4 o, d;
   float tm;
 };
-PTD PathStart start_path(const DevPaths& P, const RenderConsts& rc, uint32_t p, uint32_t s, uint32_t frame,
-                         uint32_t pix, bool batch, uint32_t sid) {
+PTD PathStart start_path(const DevPaths& P, const RenderConsts& rc, uint32_t p, uint32_t s0, uint32_t frame,
+                         uint32_t r, bool batch, uint32_t sid) {
   const PathState S = P.st[0];
-  uint32_t x = pix % rc.W, y = pix / rc.W;
-  uint32_t seed = tea64(rc.W * y + x, frame);
+  uint32_t x, y;
+  // (radiance-cache batches keep row order: the order of the paths is that
+  // of the training records)
+  if (rc.flags & PT_FLAG_RADIANCE_CACHE) {
+    y = r / rc.W;
+    x = r - y * rc.W;
+  } else {
+    tile_pixel(r, rc.W, rc.H, x, y);
+  }
+  const uint32_t pix = rc.W * y + x, s = s0 + pix;
+  uint32_t seed = tea64(pix, frame);
   float u = ((float)x + rnd(seed)) / (float)rc.W;
   float v = ((float)y + rnd(seed)) / (float)rc.H;
   const DevCamera& c = rc.cam;
@@ -259,10 +291,10 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(extend_wa
             else hi = mid - 1;
           }
           const uint32_t sid = bs.scene[lo];
-          ps = start_path(P, bs.rcs[sid], i, s, bs.frame[lo], s - bs.off[lo], true, sid);
+          ps = start_path(P, bs.rcs[sid], i, bs.off[lo], bs.frame[lo], s - bs.off[lo], true, sid);
         } else {
           const uint32_t f = s / rc.WH;
-          ps = start_path(P, rc, i, s, rc.frame0 + f, s - f * rc.WH, false, 0u);
+          ps = start_path(P, rc, i, f * rc.WH, rc.frame0 + f, s - f * rc.WH, false, 0u);
         }
         o = ps.o;
         d = ps.d;
