@@ -282,9 +282,13 @@ struct Tracer {
     }
   }
 
+  PTD bool at_node() const { return have && !(ref & LEAF_BIT); }
+
+  // the entry in hand, from the stack when there is none; false: the ray is
+  // done
   template <class ST>
-  PTD bool step(const DevScene& sc, ST& st, TraceCounts& cnt) {
-    if (!have) {
+  PTD bool next(const DevScene& sc, ST& st) {
+    while (!have) {
       if (cur >= 0 && st.sp == base_sp) {
         cur = -1;
         node_base = sc.tlas_root;
@@ -296,118 +300,151 @@ struct Tracer {
       if (st.sp == 0) return false;
       float etn;
       st.pop(ref, etn);
-      if (etn > h.t) return true;
+      have = !(etn > h.t);
     }
+    return true;
+  }
+
+  // One trip of every lane in it: an internal node, in scenes with meshes
+  // again while at least NODE_LANES lanes are at one, then a leaf or instance
+  // entry of the lanes that hold one.  Returns false once the ray is done.
+  //
+  // A triangle leaf (two tests) takes twice a node's instructions and an
+  // instance entry as many; entered at once, they ran for the few lanes that
+  // were at one while the others waited (13 of 64 lanes busy per instruction
+  // after the first bounce).  Nodes first, the leaves of several lanes meet:
+  // mesh still at 96 spp 64.0 -> 59.7 ms with 8 lanes (59.2 with 16, 59.9
+  // with 32), 16 scenes in a batch 61.0 -> 58.9 (59.5, 60.4) ms, next-week
+  // scene 3.65 -> 3.57 (3.61, 3.70) ms.  Scenes without meshes, whose leaves
+  // are cheap and nodes few, lose by the extra vote: Cornell box 10.07 ->
+  // 10.22 ms, random spheres 1.66 -> 1.70 ms.
+  static constexpr int NODE_LANES = 8;
+  template <class ST>
+  PTD bool step(const DevScene& sc, ST& st, TraceCounts& cnt) {
+    bool run;
+    do {
+      if (at_node()) node(sc, st, cnt);
+      run = next(sc, st);
+    } while (MESH && __popcll(__ballot(run && at_node())) >= NODE_LANES);
+    if (!run || at_node()) return run;
+    return leaf(sc, st, cnt);
+  }
+
+  // the leaf or instance entry in hand; false when an any-hit query ends here
+  template <class ST>
+  PTD bool leaf(const DevScene& sc, ST& st, TraceCounts& cnt) {
     have = false;
-    if (ref & LEAF_BIT) {
-      uint32_t first = ref & 0x0FFFFFFFu;
-      uint32_t count = (ref >> 28) & 7u;
-      if (cur < 0) {
-        if (FAST && count == 0) return true;  // an empty slot (a ray of NaNs)
-        // enter the instance at top-level position `first`
-        const uint4* ir = sc.insts + (size_t)first * 8;
-        float4 w0 = as_f4(ir[0]);
-        float4 w1 = as_f4(ir[1]);
-        float4 w2 = as_f4(ir[2]);
-        uint4 info = ir[3];
-        if (COUNT) cnt.insts++;
-        node_base = info.x;
-        prim_base = info.y;
-        kind = info.z & 0xFFu;
-        // the object-space ray is formed for every instance and kept where
-        // the instance has a transform: formed behind a branch on that flag,
-        // the matrix would be loaded only after the flag arrives (a second
-        // memory round trip per instance entry)
-        // (component selects: a select of whole structs keeps this state
-        // in scratch memory)
-        const bool xf = (info.z >> 8) != 0;
-        const v3 xo = xf_point(w0, w1, w2, o), xd = xf_vector(w0, w1, w2, d);
-        ro = mk3(xf ? xo.x : o.x, xf ? xo.y : o.y, xf ? xo.z : o.z);
-        rd = mk3(xf ? xd.x : d.x, xf ? xd.y : d.y, xf ? xd.z : d.z);
-        moved = xf;
-        if (xf) setup();
-        if (MESH && kind == PT_GEOM_MESH) tr = tri_setup(rd);
-        cur = (int)first;
-        base_sp = st.sp;
-        ref = 0u;  // the bottom-level root, next
-        have = true;
-        return true;
-      }
-      if (MESH && kind == PT_GEOM_MESH) {
-        // triangles two at a time: both records are loaded before either
-        // test, one memory round trip per pair (a leaf holds up to 4); the
-        // candidates are still offered in leaf order
-        for (uint32_t k = 0; k < count; k += 2) {
-          const uint32_t p0 = prim_base + first + k;
-          const bool two = k + 1 < count;
-          const uint32_t p1 = two ? p0 + 1 : p0;
-          const float4 a0 = sc.tri[3 * p0], b0 = sc.tri[3 * p0 + 1], c0 = sc.tri[3 * p0 + 2];
-          const float4 a1 = sc.tri[3 * p1], b1 = sc.tri[3 * p1 + 1], c1 = sc.tri[3 * p1 + 2];
-          if (offer_tri(sc, a0, b0, c0, cnt)) return false;
-          if (two && offer_tri(sc, a1, b1, c1, cnt)) return false;
-        }
-        return true;
-      }
-      for (uint32_t k = 0; k < count; k++) {
-        uint32_t p = prim_base + first + k;
-        if (COUNT) cnt.prims++;
-        float t = FINF;
-        uint32_t orig = 0xFFFFFFFFu;
-        if (SPH && kind == PT_GEOM_SPHERES) {
-          t = isect_sphere(sc.sph[p], ro, rd, tmin);
-        } else if (RECT && kind == PT_GEOM_RECTS) {
-          float4 A = sc.rect[2 * p], B = sc.rect[2 * p + 1];
-          const int axis = (int)__float_as_uint(B.y);
-          if (KEEP_INV) {
-            t = isect_rect(A, B.x, axis, ro, rd, axis == 0 ? rinv.x : (axis == 1 ? rinv.y : rinv.z));
-          } else {
-            t = isect_rect(A, B.x, axis, ro, rd, 1.0f / (axis == 0 ? rd.x : (axis == 1 ? rd.y : rd.z)));
-          }
-          orig = __float_as_uint(B.w);
-        } else if (BOX && kind == PT_GEOM_BOXES) {
-          float4 lo = sc.box[2 * p], hi = sc.box[2 * p + 1];
-          t = isect_box(mk3(lo), mk3(hi), ro, exact_inv(), tmin);
-          orig = __float_as_uint(lo.w);
-        } else if (EXT && kind == PT_GEOM_VOLUMES) {
-          float4 A = sc.vol[2 * p], B = sc.vol[2 * p + 1];
-          orig = __float_as_uint(B.w) & 0x7FFFFFFFu;
-          t = isect_volume(A, B, ro, rd, tmin, vol_xi(vseed, orig, (uint32_t)inst_at(sc, cur)));
-        } else if (EXT && kind == PT_GEOM_CYLINDERS) {
-          float4 A = sc.cyl[2 * p], B = sc.cyl[2 * p + 1];
-          orig = __float_as_uint(B.w);
-          t = isect_cylinder(A, B, ro, rd, tmin);
-        } else if (EXT && kind == PT_GEOM_MOVING_SPHERES) {
-          float4 A = sc.mov[3 * p], B = sc.mov[3 * p + 1], C = sc.mov[3 * p + 2];
-          v3 c = moving_center(A, B, C, time);
-          orig = __float_as_uint(B.w);
-          t = isect_sphere(make_float4(c.x, c.y, c.z, A.w), ro, rd, tmin);
-        } else if (MESH) {
-          float4 a = sc.tri[3 * p], b = sc.tri[3 * p + 1], c = sc.tri[3 * p + 2];
-          float b1, b2;
-          if (!tri_test(tr, ro, mk3(a), mk3(b), mk3(c), t, b1, b2)) t = FINF;
-          orig = __float_as_uint(a.w);
-        }
-        if (!(t > tmin)) continue;
-        bool take = t < h.t;
-        if (!take && t == h.t && h.pos >= 0) {
-          if (SPH && kind == PT_GEOM_SPHERES) orig = sc.sph_idx[p];
-          take = wins_tie(sc, (int)orig);
-        }
-        if (take) {
-          if (SPH && kind == PT_GEOM_SPHERES && orig == 0xFFFFFFFFu) orig = sc.sph_idx[p];
-          h.t = t;
-          h.prim = (int)orig;
-          h.pos = cur;
-          if (ANY && any_hit) return false;
-        }
+    uint32_t first = ref & 0x0FFFFFFFu;
+    uint32_t count = (ref >> 28) & 7u;
+    if (cur < 0) {
+      if (FAST && count == 0) return true;  // an empty slot (a ray of NaNs)
+      // enter the instance at top-level position `first`
+      const uint4* ir = sc.insts + (size_t)first * 8;
+      float4 w0 = as_f4(ir[0]);
+      float4 w1 = as_f4(ir[1]);
+      float4 w2 = as_f4(ir[2]);
+      uint4 info = ir[3];
+      if (COUNT) cnt.insts++;
+      node_base = info.x;
+      prim_base = info.y;
+      kind = info.z & 0xFFu;
+      // the object-space ray is formed for every instance and kept where
+      // the instance has a transform: formed behind a branch on that flag,
+      // the matrix would be loaded only after the flag arrives (a second
+      // memory round trip per instance entry)
+      // (component selects: a select of whole structs keeps this state
+      // in scratch memory)
+      const bool xf = (info.z >> 8) != 0;
+      const v3 xo = xf_point(w0, w1, w2, o), xd = xf_vector(w0, w1, w2, d);
+      ro = mk3(xf ? xo.x : o.x, xf ? xo.y : o.y, xf ? xo.z : o.z);
+      rd = mk3(xf ? xd.x : d.x, xf ? xd.y : d.y, xf ? xd.z : d.z);
+      moved = xf;
+      if (xf) setup();
+      if (MESH && kind == PT_GEOM_MESH) tr = tri_setup(rd);
+      cur = (int)first;
+      base_sp = st.sp;
+      ref = 0u;  // the bottom-level root, next
+      have = true;
+      return true;
+    }
+    if (MESH && kind == PT_GEOM_MESH) {
+      // triangles two at a time: both records are loaded before either
+      // test, one memory round trip per pair (a leaf holds up to 4); the
+      // candidates are still offered in leaf order
+      for (uint32_t k = 0; k < count; k += 2) {
+        const uint32_t p0 = prim_base + first + k;
+        const bool two = k + 1 < count;
+        const uint32_t p1 = two ? p0 + 1 : p0;
+        const float4 a0 = sc.tri[3 * p0], b0 = sc.tri[3 * p0 + 1], c0 = sc.tri[3 * p0 + 2];
+        const float4 a1 = sc.tri[3 * p1], b1 = sc.tri[3 * p1 + 1], c1 = sc.tri[3 * p1 + 2];
+        if (offer_tri(sc, a0, b0, c0, cnt)) return false;
+        if (two && offer_tri(sc, a1, b1, c1, cnt)) return false;
       }
       return true;
     }
-    // internal node
+    for (uint32_t k = 0; k < count; k++) {
+      uint32_t p = prim_base + first + k;
+      if (COUNT) cnt.prims++;
+      float t = FINF;
+      uint32_t orig = 0xFFFFFFFFu;
+      if (SPH && kind == PT_GEOM_SPHERES) {
+        t = isect_sphere(sc.sph[p], ro, rd, tmin);
+      } else if (RECT && kind == PT_GEOM_RECTS) {
+        float4 A = sc.rect[2 * p], B = sc.rect[2 * p + 1];
+        const int axis = (int)__float_as_uint(B.y);
+        if (KEEP_INV) {
+          t = isect_rect(A, B.x, axis, ro, rd, axis == 0 ? rinv.x : (axis == 1 ? rinv.y : rinv.z));
+        } else {
+          t = isect_rect(A, B.x, axis, ro, rd, 1.0f / (axis == 0 ? rd.x : (axis == 1 ? rd.y : rd.z)));
+        }
+        orig = __float_as_uint(B.w);
+      } else if (BOX && kind == PT_GEOM_BOXES) {
+        float4 lo = sc.box[2 * p], hi = sc.box[2 * p + 1];
+        t = isect_box(mk3(lo), mk3(hi), ro, exact_inv(), tmin);
+        orig = __float_as_uint(lo.w);
+      } else if (EXT && kind == PT_GEOM_VOLUMES) {
+        float4 A = sc.vol[2 * p], B = sc.vol[2 * p + 1];
+        orig = __float_as_uint(B.w) & 0x7FFFFFFFu;
+        t = isect_volume(A, B, ro, rd, tmin, vol_xi(vseed, orig, (uint32_t)inst_at(sc, cur)));
+      } else if (EXT && kind == PT_GEOM_CYLINDERS) {
+        float4 A = sc.cyl[2 * p], B = sc.cyl[2 * p + 1];
+        orig = __float_as_uint(B.w);
+        t = isect_cylinder(A, B, ro, rd, tmin);
+      } else if (EXT && kind == PT_GEOM_MOVING_SPHERES) {
+        float4 A = sc.mov[3 * p], B = sc.mov[3 * p + 1], C = sc.mov[3 * p + 2];
+        v3 c = moving_center(A, B, C, time);
+        orig = __float_as_uint(B.w);
+        t = isect_sphere(make_float4(c.x, c.y, c.z, A.w), ro, rd, tmin);
+      } else if (MESH) {
+        float4 a = sc.tri[3 * p], b = sc.tri[3 * p + 1], c = sc.tri[3 * p + 2];
+        float b1, b2;
+        if (!tri_test(tr, ro, mk3(a), mk3(b), mk3(c), t, b1, b2)) t = FINF;
+        orig = __float_as_uint(a.w);
+      }
+      if (!(t > tmin)) continue;
+      bool take = t < h.t;
+      if (!take && t == h.t && h.pos >= 0) {
+        if (SPH && kind == PT_GEOM_SPHERES) orig = sc.sph_idx[p];
+        take = wins_tie(sc, (int)orig);
+      }
+      if (take) {
+        if (SPH && kind == PT_GEOM_SPHERES && orig == 0xFFFFFFFFu) orig = sc.sph_idx[p];
+        h.t = t;
+        h.prim = (int)orig;
+        h.pos = cur;
+        if (ANY && any_hit) return false;
+      }
+    }
+    return true;
+  }
+
+  template <class ST>
+  PTD void node(const DevScene& sc, ST& st, TraceCounts& cnt) {
     if constexpr (FAST) {
       node_fast(sc, st);
-      return true;
+      return;
     }
+    have = false;
     if (COUNT) cnt.nodes++;
     const uint4* nd = sc.nodes + (size_t)(node_base + ref) * 8;
     uint4 q0 = nd[0], q1 = nd[1], q2 = nd[2], q3 = nd[3], q4 = nd[4], q5 = nd[5], q6 = nd[6];
@@ -449,7 +486,6 @@ struct Tracer {
       }
     }
     if (nh > 0) st.sp += nh - 1;
-    return true;
   }
 };
 
