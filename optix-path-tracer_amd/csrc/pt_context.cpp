@@ -69,17 +69,12 @@ struct pt_context {
   std::vector<pt_cylinder_desc> cylinders;
   std::vector<pt_moving_sphere_desc> moving;
   struct MeshHost {
-    std::vector<float> v, n, uv;
-    std::vector<uint32_t> idx;
-    std::vector<int32_t> fmat;
-    std::vector<int32_t> fidx;
-    int32_t mat;
+    uint32_t nv, ntri;  // vertices and triangles; the arrays live on the device
   };
   std::vector<MeshHost> meshes;
   std::vector<pt_instance_desc> instances;
   std::vector<pt_material_desc> materials;
   std::vector<pt_texture_desc> textures;
-  std::vector<std::vector<float>> texels;
   std::vector<pt_light_desc> lights;
   pt_miss_desc miss{};
 
@@ -239,6 +234,41 @@ hipError_t upload(pt_context* c, std::vector<DevBuf>& list, T** out, const void*
     if (e != hipSuccess) return e;
   }
   *out = static_cast<T*>(p);
+  return hipSuccess;
+}
+
+// A caller's array and its place (in bytes) in a device array.
+struct Part {
+  const void* src;
+  uint64_t off, bytes;
+};
+// Copies of ascending parts: large ones straight from the caller's memory,
+// runs of small neighbours gathered into one copy (a copy of its own for each
+// of a thousand small meshes would cost 10 us each).  `gathered` holds the
+// gathered runs; both they and the parts are read until the stream is
+// synchronised.
+hipError_t upload_parts(pt_context* c, void* dst, const std::vector<Part>& parts,
+                        std::vector<std::vector<uint8_t>>& gathered) {
+  constexpr uint64_t SMALL = 256 * 1024;
+  for (size_t i = 0; i < parts.size();) {
+    const void* src = parts[i].src;
+    const uint64_t off = parts[i].off;
+    uint64_t bytes = parts[i].bytes;
+    size_t j = i + 1;
+    while (bytes < SMALL && j < parts.size() && parts[j].bytes < SMALL && parts[j].off == off + bytes) bytes += parts[j++].bytes;
+    if (j > i + 1) {
+      gathered.emplace_back();
+      auto& g = gathered.back();
+      g.reserve(bytes);
+      for (size_t k = i; k < j; k++) g.insert(g.end(), (const uint8_t*)parts[k].src, (const uint8_t*)parts[k].src + parts[k].bytes);
+      src = g.data();
+    }
+    if (bytes) {
+      const hipError_t e = hipMemcpyAsync((char*)dst + off, src, bytes, hipMemcpyHostToDevice, c->stream);
+      if (e != hipSuccess) return e;
+    }
+    i = j;
+  }
   return hipSuccess;
 }
 
@@ -531,34 +561,11 @@ pt_status pt_set_scene(pt_context* c, const pt_scene_desc* d) {
   c->cylinders.assign(d->cylinders, d->cylinders + d->num_cylinders);
   c->moving.assign(d->moving_spheres, d->moving_spheres + d->num_moving_spheres);
   c->meshes.clear();
-  for (uint32_t i = 0; i < d->num_meshes; i++) {
-    const pt_mesh_desc& m = d->meshes[i];
-    pt_context::MeshHost h;
-    h.v.assign(m.vertices, m.vertices + 3ull * m.num_vertices);
-    if (m.normals) h.n.assign(m.normals, m.normals + 3ull * m.num_vertices);
-    if (m.uvs) h.uv.assign(m.uvs, m.uvs + 2ull * m.num_vertices);
-    h.idx.assign(m.indices, m.indices + 3ull * m.num_triangles);
-    if (m.face_materials) h.fmat.assign(m.face_materials, m.face_materials + m.num_triangles);
-    if (m.face_indices) h.fidx.assign(m.face_indices, m.face_indices + m.num_triangles);
-    h.mat = m.material;
-    c->meshes.push_back(std::move(h));
-  }
+  for (uint32_t i = 0; i < d->num_meshes; i++) c->meshes.push_back({d->meshes[i].num_vertices, d->meshes[i].num_triangles});
   c->instances.assign(d->instances, d->instances + d->num_instances);
   c->materials.assign(d->materials, d->materials + d->num_materials);
   c->textures.assign(d->textures, d->textures + d->num_textures);
-  c->texels.clear();
-  for (auto& t : c->textures) {
-    std::vector<float> tx;
-    if (t.type == PT_TEX_IMAGE) tx.assign(t.texels, t.texels + 4ull * t.width * t.height);
-    if (t.type == PT_TEX_NOISE) tx.assign(t.texels, t.texels + PT_NOISE_FLOATS);
-    if (t.type == PT_TEX_GRADIENT) tx.assign(t.texels, t.texels + 12);
-    if (t.type == PT_TEX_VECTOR) {
-      tx.assign(t.texels, t.texels + t.width);
-      tx.resize((tx.size() + 3) / 4 * 4, 0.f);  // whole float4 texels
-    }
-    c->texels.push_back(std::move(tx));
-    t.texels = nullptr;
-  }
+  for (auto& t : c->textures) t.texels = nullptr;
   c->lights.assign(d->lights, d->lights + d->num_lights);
   c->miss = d->miss;
   {
@@ -626,29 +633,28 @@ pt_status pt_set_scene(pt_context* c, const pt_scene_desc* d) {
     mov_mat[i] = q.material;
   }
   std::vector<DevMesh> dmesh;
-  std::vector<float4> vtx, nrm;
-  std::vector<float2> uv;
-  std::vector<uint4> idx;
   std::vector<int32_t> fmat, fidx;
-  for (auto& m : c->meshes) {
+  std::vector<Part> vparts, nparts, uparts, iparts;
+  uint64_t nv = 0, nt = 0;
+  for (uint32_t i = 0; i < d->num_meshes; i++) {
+    const pt_mesh_desc& m = d->meshes[i];
     DevMesh dm{};
-    uint32_t nv = (uint32_t)(m.v.size() / 3);
-    dm.vbase = (uint32_t)vtx.size();
-    dm.ibase = (uint32_t)idx.size();
-    dm.ntri = (uint32_t)(m.idx.size() / 3);
-    dm.has_n = !m.n.empty();
-    dm.has_uv = !m.uv.empty();
-    dm.mat = m.mat;
-    dm.fmat_base = m.fmat.empty() ? -1 : (int32_t)fmat.size();
-    dm.fidx_base = m.fidx.empty() ? -1 : (int32_t)fidx.size();
-    fidx.insert(fidx.end(), m.fidx.begin(), m.fidx.end());
-    for (uint32_t k = 0; k < nv; k++) {
-      vtx.push_back(make_float4(m.v[3 * k], m.v[3 * k + 1], m.v[3 * k + 2], 0.f));
-      nrm.push_back(dm.has_n ? make_float4(m.n[3 * k], m.n[3 * k + 1], m.n[3 * k + 2], 0.f) : make_float4(0, 0, 0, 0));
-      uv.push_back(dm.has_uv ? make_float2(m.uv[2 * k], m.uv[2 * k + 1]) : make_float2(0, 0));
-    }
-    for (uint32_t k = 0; k < dm.ntri; k++) idx.push_back(make_uint4(m.idx[3 * k], m.idx[3 * k + 1], m.idx[3 * k + 2], 0));
-    fmat.insert(fmat.end(), m.fmat.begin(), m.fmat.end());
+    dm.vbase = (uint32_t)nv;
+    dm.ibase = (uint32_t)nt;
+    dm.ntri = m.num_triangles;
+    dm.has_n = m.normals != nullptr;
+    dm.has_uv = m.uvs != nullptr;
+    dm.mat = m.material;
+    dm.fmat_base = m.face_materials ? (int32_t)fmat.size() : -1;
+    dm.fidx_base = m.face_indices ? (int32_t)fidx.size() : -1;
+    if (m.face_indices) fidx.insert(fidx.end(), m.face_indices, m.face_indices + m.num_triangles);
+    if (m.face_materials) fmat.insert(fmat.end(), m.face_materials, m.face_materials + m.num_triangles);
+    vparts.push_back({m.vertices, nv * 12, 12ull * m.num_vertices});
+    if (m.normals) nparts.push_back({m.normals, nv * 12, 12ull * m.num_vertices});
+    if (m.uvs) uparts.push_back({m.uvs, nv * 8, 8ull * m.num_vertices});
+    iparts.push_back({m.indices, nt * 12, 12ull * m.num_triangles});
+    nv += m.num_vertices;
+    nt += m.num_triangles;
     dmesh.push_back(dm);
   }
   std::vector<DevMaterial> mats;
@@ -657,13 +663,25 @@ pt_status pt_set_scene(pt_context* c, const pt_scene_desc* d) {
     mats.push_back(dm);
   }
   std::vector<DevTexture> texs;
-  std::vector<float4> texel_pool;
-  for (size_t i = 0; i < c->textures.size(); i++) {
-    auto& t = c->textures[i];
-    DevTexture dt{t.type, t.rgb[0], t.rgb[1], t.rgb[2], t.width, t.height, (uint32_t)texel_pool.size(), 0};
-    const auto& tx = c->texels[i];
-    for (size_t k = 0; k + 3 < tx.size(); k += 4) texel_pool.push_back(make_float4(tx[k], tx[k + 1], tx[k + 2], tx[k + 3]));
-    texs.push_back(dt);
+  std::vector<Part> tparts;
+  uint64_t ntexels = 0;  // float4 texels in the pool
+  std::vector<std::vector<float>> padded;  // vector-texture children in whole texels
+  for (uint32_t i = 0; i < d->num_textures; i++) {
+    const pt_texture_desc& t = d->textures[i];
+    texs.push_back(DevTexture{t.type, t.rgb[0], t.rgb[1], t.rgb[2], t.width, t.height, (uint32_t)ntexels, 0});
+    uint64_t floats = t.type == PT_TEX_IMAGE      ? 4ull * t.width * t.height
+                      : t.type == PT_TEX_NOISE    ? (uint64_t)PT_NOISE_FLOATS
+                      : t.type == PT_TEX_GRADIENT ? 12ull
+                                                  : 0ull;
+    const float* src = t.texels;
+    if (t.type == PT_TEX_VECTOR) {
+      padded.emplace_back(t.texels, t.texels + t.width);
+      padded.back().resize((t.width + 3ull) / 4 * 4, 0.f);
+      src = padded.back().data();
+      floats = padded.back().size();
+    }
+    if (floats) tparts.push_back({src, ntexels * 16, floats * 4});
+    ntexels += floats / 4;
   }
   std::vector<DevLight> lts, lts_plain;
   for (auto& l : c->lights) {
@@ -694,15 +712,49 @@ pt_status pt_set_scene(pt_context* c, const pt_scene_desc* d) {
     s.mov_instances += in.kind == PT_GEOM_MOVING_SPHERES ? 1u : 0u;
   }
   HIPCHK(c, upload(c, L, const_cast<DevMesh**>(&s.meshes), dmesh.data(), dmesh.size() * sizeof(DevMesh)));
-  HIPCHK(c, upload(c, L, const_cast<float4**>(&s.vtx), vtx.data(), vtx.size() * sizeof(float4)));
-  HIPCHK(c, upload(c, L, const_cast<float4**>(&s.nrm), nrm.data(), nrm.size() * sizeof(float4)));
-  HIPCHK(c, upload(c, L, const_cast<float2**>(&s.uv), uv.data(), uv.size() * sizeof(float2)));
-  HIPCHK(c, upload(c, L, const_cast<uint4**>(&s.idx), idx.data(), idx.size() * sizeof(uint4)));
+  {
+    // vertices, normals and index triples travel as the caller's packed
+    // words and are widened to 16-byte records on the GPU
+    std::vector<DevBuf> raw;
+    std::vector<std::vector<uint8_t>> gathered;  // read by copies until the synchronisation
+    uint32_t *wv = nullptr, *wn = nullptr, *wi = nullptr;
+    hipError_t e = hipSuccess;
+    if ((e = dalloc(L, (void**)&s.vtx, nv * sizeof(float4))) || (e = dalloc(L, (void**)&s.nrm, nv * sizeof(float4))) ||
+        (e = dalloc(L, (void**)&s.uv, nv * sizeof(float2))) || (e = dalloc(L, (void**)&s.idx, nt * sizeof(uint4))) ||
+        (e = dalloc(raw, (void**)&wv, nv * 12)) || (e = dalloc(raw, (void**)&wi, nt * 12)) ||
+        (!nparts.empty() && (e = dalloc(raw, (void**)&wn, nv * 12)))) {
+      dfree(raw);
+      return hip_fail(c, e, "hipMalloc (meshes)");
+    }
+    if (nparts.size() < d->num_meshes) {  // meshes without normals hold zeros
+      if (wn) launch_fill_u32(wn, nv * 3, 0u, c->stream);
+      else launch_fill_u32((uint32_t*)s.nrm, nv * 4, 0u, c->stream);
+    }
+    if (nv && uparts.size() < d->num_meshes) launch_fill_u32((uint32_t*)s.uv, nv * 2, 0u, c->stream);
+    e = upload_parts(c, wv, vparts, gathered);
+    if (e == hipSuccess) e = upload_parts(c, wi, iparts, gathered);
+    if (e == hipSuccess && wn) e = upload_parts(c, wn, nparts, gathered);
+    if (e == hipSuccess) e = upload_parts(c, (void*)s.uv, uparts, gathered);
+    if (e == hipSuccess) {
+      launch_widen3(wv, nv, (uint4*)s.vtx, c->stream);
+      launch_widen3(wi, nt, (uint4*)s.idx, c->stream);
+      if (wn) launch_widen3(wn, nv, (uint4*)s.nrm, c->stream);
+    }
+    const hipError_t es = hipStreamSynchronize(c->stream);
+    dfree(raw);
+    if (e != hipSuccess || (e = es) != hipSuccess) return hip_fail(c, e, "upload meshes");
+  }
   HIPCHK(c, upload(c, L, const_cast<int32_t**>(&s.fmat), fmat.data(), fmat.size() * 4));
   HIPCHK(c, upload(c, L, const_cast<int32_t**>(&s.fidx), fidx.data(), fidx.size() * 4));
   HIPCHK(c, upload(c, L, const_cast<DevMaterial**>(&s.mats), mats.data(), mats.size() * sizeof(DevMaterial)));
   HIPCHK(c, upload(c, L, const_cast<DevTexture**>(&s.texs), texs.data(), texs.size() * sizeof(DevTexture)));
-  HIPCHK(c, upload(c, L, const_cast<float4**>(&s.texels), texel_pool.data(), texel_pool.size() * sizeof(float4)));
+  {
+    std::vector<std::vector<uint8_t>> gathered;
+    hipError_t e = dalloc(L, (void**)&s.texels, ntexels * sizeof(float4));
+    if (e == hipSuccess) e = upload_parts(c, (void*)s.texels, tparts, gathered);
+    const hipError_t es = hipStreamSynchronize(c->stream);
+    if (e != hipSuccess || (e = es) != hipSuccess) return hip_fail(c, e, "upload textures");
+  }
   HIPCHK(c, upload(c, L, const_cast<DevLight**>(&s.lights), lts.data(), lts.size() * sizeof(DevLight)));
   HIPCHK(c, upload(c, L, const_cast<DevLight**>(&s.lights_plain), lts_plain.data(),
                    lts_plain.size() * sizeof(DevLight)));
@@ -764,7 +816,7 @@ pt_status pt_build_accel(pt_context* c, pt_accel_stats* out) {
   uint32_t pool_n[7] = {0, 0, 0, 0, 0, 0, 0};
   for (size_t i = 0; i < c->instances.size(); i++) {
     const auto& in = c->instances[i];
-    uint32_t count = in.kind == PT_GEOM_MESH ? (uint32_t)(c->meshes[in.first].idx.size() / 3) : in.count;
+    uint32_t count = in.kind == PT_GEOM_MESH ? c->meshes[in.first].ntri : in.count;
     auto key = std::make_tuple((int)in.kind, in.first, count);
     auto it = blas_of.find(key);
     if (it == blas_of.end()) {
@@ -846,8 +898,8 @@ pt_status pt_build_accel(pt_context* c, pt_accel_stats* out) {
         // device mesh table offsets are computed in set_scene in mesh order
         uint32_t vbase = 0, ibase = 0;
         for (uint32_t m = 0; m < bi.first; m++) {
-          vbase += (uint32_t)(c->meshes[m].v.size() / 3);
-          ibase += (uint32_t)(c->meshes[m].idx.size() / 3);
+          vbase += c->meshes[m].nv;
+          ibase += c->meshes[m].ntri;
         }
         launch_bounds_tris(s.vtx + vbase, s.idx + ibase, n, sb.lo, sb.hi, c->stream);
       }
@@ -897,8 +949,8 @@ pt_status pt_build_accel(pt_context* c, pt_accel_stats* out) {
       default: {
         uint32_t vbase = 0, ibase = 0;
         for (uint32_t m = 0; m < bi.first; m++) {
-          vbase += (uint32_t)(c->meshes[m].v.size() / 3);
-          ibase += (uint32_t)(c->meshes[m].idx.size() / 3);
+          vbase += c->meshes[m].nv;
+          ibase += c->meshes[m].ntri;
         }
         launch_gather_tris(s.vtx + vbase, s.idx + ibase, ord, n, tri + 3ull * bi.prim_base, c->stream);
       }

@@ -101,6 +101,8 @@ void launch_accumulate(const DevPaths& P, const RenderConsts& rc, uint32_t nfram
                        int grid, hipStream_t st);
 void launch_display(const double* accum, uint32_t npix, uint32_t frames, uchar4* rgba, int grid, hipStream_t st);
 void launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t st);
+// n packed triples of words -> (x, y, z, 0)
+void launch_widen3(const uint32_t* src, uint64_t n, uint4* dst, hipStream_t st);
 void launch_fill_f64(double* p, uint64_t n, double v, hipStream_t st);
 
 // radiance-cache network (pt_mlp.hip)

