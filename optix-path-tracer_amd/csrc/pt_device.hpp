@@ -18,6 +18,14 @@ namespace pt {
 
 #define PTD __device__ __forceinline__
 
+// A pointer into device memory that was itself loaded from memory (a batch's
+// scene table): the compiler cannot tell that it is global and would load
+// through it with flat instructions, which also count as LDS accesses.
+template <class T>
+PTD const T* gp(const T* p) {
+  return (const T*)(const __attribute__((address_space(1))) T*)p;
+}
+
 constexpr float PI_F = 3.141592654f;  // programs/common.hpp:18
 constexpr float FINF = __builtin_huge_valf();
 constexpr float SLAB_FAR_SCALE = 1.00000024f;  // 1 + 2^-22, conservative slab test

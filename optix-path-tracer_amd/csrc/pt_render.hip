@@ -268,7 +268,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(extend_wa
   const PathState S = P.st[in];
   uint32_t bc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   TraceCounts c{0, 0, 0};
-  constexpr bool REFILL = PT_EXTEND_REFILL > 0 && !START && !MULTI && (KINDS & 8) != 0;
+  constexpr bool REFILL = PT_EXTEND_REFILL > 0 && !START && (KINDS & 8) != 0;
   if (REFILL) {
     // Bounce rays in scenes with meshes differ widely in length (the sky
     // after one node, a mesh after dozens): each lane keeps tracing paths
@@ -277,20 +277,24 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(extend_wa
     // set-ups per refill).  Every path is traced exactly as alone, so hits
     // and counts do not depend on which lane takes it.  (Scenes of a few
     // primitives, whose rays are all short, run faster in lock-step: the
-    // lanes' steps stay alike.)
-    Tracer<COUNT, EXT, KINDS> tr;
-    uint32_t j = __lane_id();
+    // lanes' steps stay alike.)  In a batch of scenes each lane keeps its
+    // scene (16 scenes 59.1 -> 58.7 ms per pass, and 57.8 ms with the node
+    // array's address kept per ray and the table's pointers known as global).
+    Tracer<COUNT, EXT, KINDS, false, MULTI> tr;
+    uint32_t j = __lane_id(), sid = 0;
+    auto scene = [&]() -> const DevScene& { return MULTI ? scenes[sid] : sc0; };
     bool busy = j < n;
     uint32_t next = 64;  // wave-uniform: the next position to hand out
     auto take = [&](uint32_t jj) {
       const uint32_t i = g.pos(jj);
       const float4 o = S.o[i], d = S.d[i];
-      const float tm = (EXT && sc0.mov_instances) ? P.ptime[__float_as_uint(d.w) & SLOT_MASK] : 0.f;
-      tr.begin(sc0, mk3(o), mk3(d), tmin, FINF, st, __float_as_uint(o.w), tm);
+      sid = __float_as_uint(o.w) >> 24;
+      const float tm = (EXT && scene().mov_instances) ? P.ptime[__float_as_uint(d.w) & SLOT_MASK] : 0.f;
+      tr.begin(scene(), mk3(o), mk3(d), tmin, FINF, st, __float_as_uint(o.w), tm);
     };
     if (busy) take(j);
     while (true) {
-      if (busy && !tr.step(sc0, st, c)) {
+      if (busy && !tr.step(scene(), st, c)) {
         P.hit[g.pos(j)] = make_float4(tr.h.t, __int_as_float(tr.h.pos), __int_as_float(tr.h.prim), 0.f);
         busy = false;
       }
@@ -319,7 +323,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(extend_wa
         uint32_t key = 0xFFu;
         if (jj < n) {
           const uint32_t i = g.pos(jj);
-          key = material_key(sc0, P.hit[i]);
+          key = material_key(MULTI ? scenes[__float_as_uint(S.o[i].w) >> 24] : sc0, P.hit[i]);
           P.keys[i] = key;
         }
 #pragma unroll

@@ -21,7 +21,7 @@ struct HitRec {
 template <int KINDS = 15, bool EXT = true>
 PTD HitRec hit_record(const DevScene& sc, int inst_pos, int prim, float t, v3 o, v3 d, bool need_uv_hint,
                       float time = 0.f) {
-  const uint4* ir = sc.insts + (size_t)inst_pos * 8;
+  const uint4* ir = gp(sc.insts) + (size_t)inst_pos * 8;
   float4 w0 = as_f4(ir[0]), w1 = as_f4(ir[1]), w2 = as_f4(ir[2]);
   uint4 info = ir[3];
   uint32_t kind = info.z & 0xFFu;
@@ -39,8 +39,8 @@ PTD HitRec hit_record(const DevScene& sc, int inst_pos, int prim, float t, v3 o,
   v3 hp = ro, n = mk3(0.f, 1.f, 0.f);  // every kind that occurs sets both
   r.mat = 0;
   if ((KINDS & 1) && kind == PT_GEOM_SPHERES) {
-    float4 s = sc.sph_o[prim];
-    r.mat = sc.sph_mat[prim];
+    float4 s = gp(sc.sph_o)[prim];
+    r.mat = gp(sc.sph_mat)[prim];
     hp = ro + t * rd;
     n = (hp - mk3(s)) / s.w;
     if (need_uv_hint) {
@@ -50,8 +50,8 @@ PTD HitRec hit_record(const DevScene& sc, int inst_pos, int prim, float t, v3 o,
       r.v = (theta + PI_F / 2.f) / PI_F;
     }
   } else if ((KINDS & 2) && kind == PT_GEOM_RECTS) {
-    float4 A = sc.rect_o[2 * prim], B = sc.rect_o[2 * prim + 1];
-    r.mat = sc.rect_mat[prim];
+    float4 A = gp(sc.rect_o)[2 * prim], B = gp(sc.rect_o)[2 * prim + 1];
+    r.mat = gp(sc.rect_mat)[prim];
     int axis = (int)__float_as_uint(B.y);
     hp = ro + t * rd;
     // aarect.cu:88-100; u, v only where a texture reads them
@@ -67,8 +67,8 @@ PTD HitRec hit_record(const DevScene& sc, int inst_pos, int prim, float t, v3 o,
     }
     if (__float_as_uint(B.z)) n = -n;
   } else if ((KINDS & 4) && kind == PT_GEOM_BOXES) {
-    float4 lo = sc.box_o[2 * prim], hi = sc.box_o[2 * prim + 1];
-    r.mat = sc.box_mat[prim];
+    float4 lo = gp(sc.box_o)[2 * prim], hi = gp(sc.box_o)[2 * prim + 1];
+    r.mat = gp(sc.box_mat)[prim];
     hp = ro + t * rd;
     // the slab distances exactly as the intersection formed them
     v3 rinv = mk3(1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z);
@@ -79,14 +79,14 @@ PTD HitRec hit_record(const DevScene& sc, int inst_pos, int prim, float t, v3 o,
     n = pos - neg;
   } else if (EXT && kind == PT_GEOM_CYLINDERS) {
     // cylinder.cu:70-97: radial normal, no uv
-    float4 A = sc.cyl_o[2 * prim];
-    r.mat = sc.cyl_mat[prim];
+    float4 A = gp(sc.cyl_o)[2 * prim];
+    r.mat = gp(sc.cyl_mat)[prim];
     hp = ro + t * rd;
     n = normalize(hp - mk3(A.x, hp.y, A.z));
   } else if (EXT && kind == PT_GEOM_MOVING_SPHERES) {
     // moving_sphere.cu:78-91 with the center at the path's time, in object space
-    float4 A = sc.mov_o[3 * prim], B = sc.mov_o[3 * prim + 1], C = sc.mov_o[3 * prim + 2];
-    r.mat = sc.mov_mat[prim];
+    float4 A = gp(sc.mov_o)[3 * prim], B = gp(sc.mov_o)[3 * prim + 1], C = gp(sc.mov_o)[3 * prim + 2];
+    r.mat = gp(sc.mov_mat)[prim];
     v3 c = moving_center(A, B, C, time);
     hp = ro + t * rd;
     n = (hp - c) / A.w;
@@ -98,13 +98,13 @@ PTD HitRec hit_record(const DevScene& sc, int inst_pos, int prim, float t, v3 o,
     }
   } else if (EXT && kind == PT_GEOM_VOLUMES) {
     // volume_sphere.cu:88-100: the scatter point, normal +X, no uv
-    r.mat = sc.vol_mat[prim];
+    r.mat = gp(sc.vol_mat)[prim];
     hp = ro + t * rd;
     n = mk3(1.f, 0.f, 0.f);
   } else if (KINDS & 8) {
-    const DevMesh& m = sc.meshes[ir[7].z];
-    uint4 ix = sc.idx[m.ibase + prim];
-    v3 a = mk3(sc.vtx[m.vbase + ix.x]), b = mk3(sc.vtx[m.vbase + ix.y]), c = mk3(sc.vtx[m.vbase + ix.z]);
+    const DevMesh& m = gp(sc.meshes)[ir[7].z];
+    uint4 ix = gp(sc.idx)[m.ibase + prim];
+    v3 a = mk3(gp(sc.vtx)[m.vbase + ix.x]), b = mk3(gp(sc.vtx)[m.vbase + ix.y]), c = mk3(gp(sc.vtx)[m.vbase + ix.z]);
     TriRay tr = tri_setup(rd);
     float tt = 0.f, b1 = 0.f, b2 = 0.f;
     tri_test(tr, ro, a, b, c, tt, b1, b2);
@@ -112,15 +112,15 @@ PTD HitRec hit_record(const DevScene& sc, int inst_pos, int prim, float t, v3 o,
     hp = a * b0 + b * b1 + c * b2;
     n = cross(b - a, c - a);
     if (m.has_n) {
-      n = mk3(sc.nrm[m.vbase + ix.x]) * b0 + mk3(sc.nrm[m.vbase + ix.y]) * b1 + mk3(sc.nrm[m.vbase + ix.z]) * b2;
+      n = mk3(gp(sc.nrm)[m.vbase + ix.x]) * b0 + mk3(gp(sc.nrm)[m.vbase + ix.y]) * b1 + mk3(gp(sc.nrm)[m.vbase + ix.z]) * b2;
     }
     if (m.has_uv) {
-      float2 ua = sc.uv[m.vbase + ix.x], ub = sc.uv[m.vbase + ix.y], uc = sc.uv[m.vbase + ix.z];
+      float2 ua = gp(sc.uv)[m.vbase + ix.x], ub = gp(sc.uv)[m.vbase + ix.y], uc = gp(sc.uv)[m.vbase + ix.z];
       r.u = ua.x * b0 + ub.x * b1 + uc.x * b2;
       r.v = ua.y * b0 + ub.y * b1 + uc.y * b2;
     }
-    r.mat = m.fmat_base >= 0 ? sc.fmat[m.fmat_base + prim] : m.mat;
-    if (m.fidx_base >= 0) r.fidx = sc.fidx[m.fidx_base + prim];
+    r.mat = m.fmat_base >= 0 ? gp(sc.fmat)[m.fmat_base + prim] : m.mat;
+    if (m.fidx_base >= 0) r.fidx = gp(sc.fidx)[m.fidx_base + prim];
   }
   if (xf) {
     float4 m0 = as_f4(ir[4]), m1 = as_f4(ir[5]), m2 = as_f4(ir[6]);
@@ -145,7 +145,7 @@ PTD v3 tex_image(const DevScene& sc, const DevTexture& t, float u, float v) {
   long long i1 = (xi + 1) % W; if (i1 < 0) i1 += W;
   long long j0 = yi % H; if (j0 < 0) j0 += H;
   long long j1 = (yi + 1) % H; if (j1 < 0) j1 += H;
-  const float4* p = sc.texels + t.offset;
+  const float4* p = gp(sc.texels) + t.offset;
   v3 c00 = mk3(p[j0 * W + i0]), c10 = mk3(p[j0 * W + i1]);
   v3 c01 = mk3(p[j1 * W + i0]), c11 = mk3(p[j1 * W + i1]);
   v3 top = c00 * (1.f - fx) + c10 * fx;
@@ -187,13 +187,13 @@ PTD v3 tex_leaf(const DevScene& sc, const DevTexture& t, float u, float v, v3 P)
   if (t.type == PT_TEX_CONSTANT) return mk3(t.r, t.g, t.b);
   if (t.type == PT_TEX_NOISE) {
     // noise_texture.cu:70-84: the axis switch falls through to the Z case
-    const float4* tab = sc.texels + t.offset;
+    const float4* tab = gp(sc.texels) + t.offset;
     float sv = psin(t.r * P.z + 5 * perlin_turb(tab, t.r * P));
     return mk3(1.f) * 0.5f * (1 + sv);
   }
   if (t.type == PT_TEX_GRADIENT) {
     // gradient_texture.cu:7-14
-    const float4* c = sc.texels + t.offset;
+    const float4* c = gp(sc.texels) + t.offset;
     v3 ud = normalize(P);
     float x = fabsf(ud.x), y = fabsf(ud.y), z = fabsf(ud.z);
     return x * mk3(c[0]) + y * mk3(c[1]) + z * mk3(c[2]);
@@ -203,28 +203,28 @@ PTD v3 tex_leaf(const DevScene& sc, const DevTexture& t, float u, float v, v3 P)
 // vector.cu:7-12: child `fidx` of a vector texture (children see index 0),
 // black when it is out of range
 PTD v3 tex_eval(const DevScene& sc, int ti, float u, float v, v3 P = mk3(0.f), int fidx = 0) {
-  if (sc.texs[ti].type == PT_TEX_VECTOR) {
-    const DevTexture& tv = sc.texs[ti];
+  if (gp(sc.texs)[ti].type == PT_TEX_VECTOR) {
+    const DevTexture& tv = gp(sc.texs)[ti];
     if (fidx < 0 || (uint32_t)fidx >= tv.w) return mk3(0.f);
-    ti = (int)reinterpret_cast<const float*>(sc.texels + tv.offset)[fidx];
+    ti = (int)reinterpret_cast<const float*>(gp(sc.texels) + tv.offset)[fidx];
   }
-  const DevTexture& t = sc.texs[ti];
+  const DevTexture& t = gp(sc.texs)[ti];
   if (t.type == PT_TEX_CHECKER) {
     // checkered_texture.cu:8-15 (odd in w, even in h)
     float sines = psin(10 * P.x) * psin(10 * P.y) * psin(10 * P.z);
-    return tex_leaf(sc, sc.texs[sines < 0 ? t.w : t.h], u, v, P);
+    return tex_leaf(sc, gp(sc.texs)[sines < 0 ? t.w : t.h], u, v, P);
   }
   return tex_leaf(sc, t, u, v, P);
 }
 // Geometric normal of a hit for normal_shader.cu:27-31: differs from the
 // hit record's (shading) normal only on meshes with vertex normals.
 PTD v3 geometric_normal(const DevScene& sc, int inst_pos, int prim, v3 n_shading) {
-  const uint4* ir = sc.insts + (size_t)inst_pos * 8;
+  const uint4* ir = gp(sc.insts) + (size_t)inst_pos * 8;
   if ((ir[3].z & 0xFFu) != PT_GEOM_MESH) return n_shading;
-  const DevMesh& m = sc.meshes[ir[7].z];
+  const DevMesh& m = gp(sc.meshes)[ir[7].z];
   if (!m.has_n) return n_shading;
-  uint4 ix = sc.idx[m.ibase + prim];
-  v3 a = mk3(sc.vtx[m.vbase + ix.x]), b = mk3(sc.vtx[m.vbase + ix.y]), c = mk3(sc.vtx[m.vbase + ix.z]);
+  uint4 ix = gp(sc.idx)[m.ibase + prim];
+  v3 a = mk3(gp(sc.vtx)[m.vbase + ix.x]), b = mk3(gp(sc.vtx)[m.vbase + ix.y]), c = mk3(gp(sc.vtx)[m.vbase + ix.z]);
   v3 n = cross(b - a, c - a);
   if ((ir[3].z >> 8) != 0) n = xf_normal(as_f4(ir[0]), as_f4(ir[1]), as_f4(ir[2]), n);
   return normalize(n);
@@ -232,13 +232,13 @@ PTD v3 geometric_normal(const DevScene& sc, int inst_pos, int prim, v3 n_shading
 
 PTD bool tex_needs_uv(const DevScene& sc, int ti) {
   if (ti < 0) return false;
-  const DevTexture& t = sc.texs[ti];
-  if (t.type == PT_TEX_CHECKER) return sc.texs[t.w].type == PT_TEX_IMAGE || sc.texs[t.h].type == PT_TEX_IMAGE;
+  const DevTexture& t = gp(sc.texs)[ti];
+  if (t.type == PT_TEX_CHECKER) return gp(sc.texs)[t.w].type == PT_TEX_IMAGE || gp(sc.texs)[t.h].type == PT_TEX_IMAGE;
   return t.type == PT_TEX_IMAGE || t.type == PT_TEX_VECTOR;  // vectors: conservatively
 }
 
 PTD Surface make_surface(const DevScene& sc, const HitRec& r) {
-  const DevMaterial& m = sc.mats[r.mat];
+  const DevMaterial& m = gp(sc.mats)[r.mat];
   Surface f;
   f.type = m.type;
   f.c0 = m.tex0 >= 0 ? tex_eval(sc, m.tex0, r.u, r.v, r.P, r.fidx) : mk3(0.f);  // the normal shader has none
@@ -291,7 +291,7 @@ PTD float env_pdf(const DevScene& sc, v3 d) {
   if (j >= (long long)sc.env_h) j = sc.env_h - 1;
   if (i < 0) i = 0;
   if (j < 0) j = 0;
-  const unsigned long long* row = sc.env_cond + (size_t)j * sc.env_w;
+  const unsigned long long* row = gp(sc.env_cond) + (size_t)j * sc.env_w;
   unsigned long long w = row[i] - (i ? row[i - 1] : 0ull);
   float st = psin(v * PI_F);
   if (w == 0 || !(st > 0.f)) return 0.f;
@@ -323,13 +323,13 @@ PTD v3 env_sample(const DevScene& sc, uint32_t& seed) {
   uint32_t r2 = lcg24(seed);
   if (sc.env_total == 0) return mk3(0.f, 1.f, 0.f);
   unsigned long long tr = scale24(sc.env_total, r1);
-  const uint32_t* gm = sc.env_guide + (size_t)sc.env_h * (ENV_GUIDE + 1);
+  const uint32_t* gm = gp(sc.env_guide) + (size_t)sc.env_h * (ENV_GUIDE + 1);
   uint32_t j = guided_index(sc.env_marg, sc.env_h, sc.env_total, tr, gm);
-  unsigned long long rprev = j ? sc.env_marg[j - 1] : 0ull;
-  unsigned long long rw = sc.env_marg[j] - rprev;
-  const unsigned long long* row = sc.env_cond + (size_t)j * sc.env_w;
+  unsigned long long rprev = j ? gp(sc.env_marg)[j - 1] : 0ull;
+  unsigned long long rw = gp(sc.env_marg)[j] - rprev;
+  const unsigned long long* row = gp(sc.env_cond) + (size_t)j * sc.env_w;
   unsigned long long tc = scale24(rw, r2);
-  uint32_t i = guided_index(row, sc.env_w, rw, tc, sc.env_guide + (size_t)j * (ENV_GUIDE + 1));
+  uint32_t i = guided_index(row, sc.env_w, rw, tc, gp(sc.env_guide) + (size_t)j * (ENV_GUIDE + 1));
   unsigned long long cprev = i ? row[i - 1] : 0ull;
   // offsets inside the texel, below 1 (a ratio of two roundings may reach it)
   const float fu = fminf((float)(tc - cprev) / (float)(row[i] - cprev), 0x1.fffffep-1f);
@@ -432,16 +432,16 @@ PTD v3 light_emission(const DevLight& l) { return mk3(l.ex, l.ey, l.ez); }
 
 // material of a hit (for the shadow-ray rule and the material sort)
 PTD int hit_material(const DevScene& sc, int inst_pos, int prim) {
-  const uint4* ir = sc.insts + (size_t)inst_pos * 8;
+  const uint4* ir = gp(sc.insts) + (size_t)inst_pos * 8;
   uint32_t kind = ir[3].z & 0xFFu;
-  if (kind == PT_GEOM_SPHERES) return sc.sph_mat[prim];
-  if (kind == PT_GEOM_RECTS) return sc.rect_mat[prim];
-  if (kind == PT_GEOM_BOXES) return sc.box_mat[prim];
-  if (kind == PT_GEOM_VOLUMES) return sc.vol_mat[prim];
-  if (kind == PT_GEOM_CYLINDERS) return sc.cyl_mat[prim];
-  if (kind == PT_GEOM_MOVING_SPHERES) return sc.mov_mat[prim];
-  const DevMesh& m = sc.meshes[ir[7].z];
-  return m.fmat_base >= 0 ? sc.fmat[m.fmat_base + prim] : m.mat;
+  if (kind == PT_GEOM_SPHERES) return gp(sc.sph_mat)[prim];
+  if (kind == PT_GEOM_RECTS) return gp(sc.rect_mat)[prim];
+  if (kind == PT_GEOM_BOXES) return gp(sc.box_mat)[prim];
+  if (kind == PT_GEOM_VOLUMES) return gp(sc.vol_mat)[prim];
+  if (kind == PT_GEOM_CYLINDERS) return gp(sc.cyl_mat)[prim];
+  if (kind == PT_GEOM_MOVING_SPHERES) return gp(sc.mov_mat)[prim];
+  const DevMesh& m = gp(sc.meshes)[ir[7].z];
+  return m.fmat_base >= 0 ? gp(sc.fmat)[m.fmat_base + prim] : m.mat;
 }
 
 }  // namespace pt

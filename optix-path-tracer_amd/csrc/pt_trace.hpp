@@ -55,7 +55,7 @@ struct HitOut {
   int pos;   // instance position in top-level order (-1: miss)
 };
 // original instance id of the instance at top-level position pos
-PTD int inst_at(const DevScene& sc, int pos) { return (int)sc.insts[(size_t)pos * 8 + 3].w; }
+PTD int inst_at(const DevScene& sc, int pos) { return (int)gp(sc.insts)[(size_t)pos * 8 + 3].w; }
 
 struct TraceCounts {
   uint32_t nodes, prims, insts;
@@ -116,6 +116,9 @@ struct Tracer {
   int cur;      // instance slot in top-level order, -1 = top level
   int base_sp;  // stack depth when the instance was entered
   uint32_t node_base, prim_base, kind;
+  // WIDE: the address of node node_base instead (a batch's kernels would
+  // fetch the node array's address from the scene's table entry at each node)
+  uint64_t node_ptr;
   bool moved;   // the instance in hand has a transform: ro, rd are its own
   // the entry in hand: the top-level root first; the nearest child of each
   // node and an instance's root are taken directly instead of through the
@@ -168,7 +171,7 @@ struct Tracer {
     tr = TriRay{0, 0.f, 0.f, 0.f};
     cur = -1;
     base_sp = 0;
-    node_base = sc.tlas_root;
+    enter_nodes(sc, sc.tlas_root);
     prim_base = 0;
     kind = 0;
     st.sp = 0;
@@ -235,10 +238,8 @@ struct Tracer {
     typedef uint32_t u4 __attribute__((ext_vector_type(4)));
     f4 nx, ny, nz, fx, fy, fz;
     u4 cr;
-    const uint32_t index = node_base + ref;
     if constexpr (WIDE) {
-      typedef const __attribute__((address_space(1))) char* gp;
-      const uint64_t p = (uint64_t)(gp)sc.nodes + ((uint64_t)index << 7);
+      const uint64_t p = node_ptr + ((uint64_t)ref << 7);
       auto ld = [&](uint32_t k) { return *(const __attribute__((address_space(1))) f4*)(p | k); };
       nx = ld(sx); fx = ld(sx ^ 16u);
       ny = ld(sy); fy = ld(sy ^ 16u);
@@ -246,7 +247,7 @@ struct Tracer {
       cr = *(const __attribute__((address_space(1))) u4*)(p + 96u);
     } else {
       const char* b = reinterpret_cast<const char*>(sc.nodes);
-      const uint32_t p = index << 7;
+      const uint32_t p = (node_base + ref) << 7;
       auto ld = [&](uint32_t k) { return *reinterpret_cast<const f4*>(b + (p | k)); };
       nx = ld(sx); fx = ld(sx ^ 16u);
       ny = ld(sy); fy = ld(sy ^ 16u);
@@ -282,6 +283,13 @@ struct Tracer {
     }
   }
 
+  PTD void enter_nodes(const DevScene& sc, uint32_t base) {
+    if (WIDE && FAST)
+      node_ptr = (uint64_t)(const __attribute__((address_space(1))) char*)(const char*)sc.nodes + ((uint64_t)base << 7);
+    else
+      node_base = base;
+  }
+
   PTD bool at_node() const { return have && !(ref & LEAF_BIT); }
 
   // the entry in hand, from the stack when there is none; false: the ray is
@@ -291,7 +299,7 @@ struct Tracer {
     while (!have) {
       if (cur >= 0 && st.sp == base_sp) {
         cur = -1;
-        node_base = sc.tlas_root;
+        enter_nodes(sc, sc.tlas_root);
         if (moved) {
           ro = o; rd = d;
           setup();
@@ -339,13 +347,13 @@ struct Tracer {
     if (cur < 0) {
       if (FAST && count == 0) return true;  // an empty slot (a ray of NaNs)
       // enter the instance at top-level position `first`
-      const uint4* ir = sc.insts + (size_t)first * 8;
+      const uint4* ir = gp(sc.insts) + (size_t)first * 8;
       float4 w0 = as_f4(ir[0]);
       float4 w1 = as_f4(ir[1]);
       float4 w2 = as_f4(ir[2]);
       uint4 info = ir[3];
       if (COUNT) cnt.insts++;
-      node_base = info.x;
+      enter_nodes(sc, info.x);
       prim_base = info.y;
       kind = info.z & 0xFFu;
       // the object-space ray is formed for every instance and kept where
@@ -375,8 +383,8 @@ struct Tracer {
         const uint32_t p0 = prim_base + first + k;
         const bool two = k + 1 < count;
         const uint32_t p1 = two ? p0 + 1 : p0;
-        const float4 a0 = sc.tri[3 * p0], b0 = sc.tri[3 * p0 + 1], c0 = sc.tri[3 * p0 + 2];
-        const float4 a1 = sc.tri[3 * p1], b1 = sc.tri[3 * p1 + 1], c1 = sc.tri[3 * p1 + 2];
+        const float4 a0 = gp(sc.tri)[3 * p0], b0 = gp(sc.tri)[3 * p0 + 1], c0 = gp(sc.tri)[3 * p0 + 2];
+        const float4 a1 = gp(sc.tri)[3 * p1], b1 = gp(sc.tri)[3 * p1 + 1], c1 = gp(sc.tri)[3 * p1 + 2];
         if (offer_tri(sc, a0, b0, c0, cnt)) return false;
         if (two && offer_tri(sc, a1, b1, c1, cnt)) return false;
       }
@@ -388,9 +396,9 @@ struct Tracer {
       float t = FINF;
       uint32_t orig = 0xFFFFFFFFu;
       if (SPH && kind == PT_GEOM_SPHERES) {
-        t = isect_sphere(sc.sph[p], ro, rd, tmin);
+        t = isect_sphere(gp(sc.sph)[p], ro, rd, tmin);
       } else if (RECT && kind == PT_GEOM_RECTS) {
-        float4 A = sc.rect[2 * p], B = sc.rect[2 * p + 1];
+        float4 A = gp(sc.rect)[2 * p], B = gp(sc.rect)[2 * p + 1];
         const int axis = (int)__float_as_uint(B.y);
         if (KEEP_INV) {
           t = isect_rect(A, B.x, axis, ro, rd, axis == 0 ? rinv.x : (axis == 1 ? rinv.y : rinv.z));
@@ -399,24 +407,24 @@ struct Tracer {
         }
         orig = __float_as_uint(B.w);
       } else if (BOX && kind == PT_GEOM_BOXES) {
-        float4 lo = sc.box[2 * p], hi = sc.box[2 * p + 1];
+        float4 lo = gp(sc.box)[2 * p], hi = gp(sc.box)[2 * p + 1];
         t = isect_box(mk3(lo), mk3(hi), ro, exact_inv(), tmin);
         orig = __float_as_uint(lo.w);
       } else if (EXT && kind == PT_GEOM_VOLUMES) {
-        float4 A = sc.vol[2 * p], B = sc.vol[2 * p + 1];
+        float4 A = gp(sc.vol)[2 * p], B = gp(sc.vol)[2 * p + 1];
         orig = __float_as_uint(B.w) & 0x7FFFFFFFu;
         t = isect_volume(A, B, ro, rd, tmin, vol_xi(vseed, orig, (uint32_t)inst_at(sc, cur)));
       } else if (EXT && kind == PT_GEOM_CYLINDERS) {
-        float4 A = sc.cyl[2 * p], B = sc.cyl[2 * p + 1];
+        float4 A = gp(sc.cyl)[2 * p], B = gp(sc.cyl)[2 * p + 1];
         orig = __float_as_uint(B.w);
         t = isect_cylinder(A, B, ro, rd, tmin);
       } else if (EXT && kind == PT_GEOM_MOVING_SPHERES) {
-        float4 A = sc.mov[3 * p], B = sc.mov[3 * p + 1], C = sc.mov[3 * p + 2];
+        float4 A = gp(sc.mov)[3 * p], B = gp(sc.mov)[3 * p + 1], C = gp(sc.mov)[3 * p + 2];
         v3 c = moving_center(A, B, C, time);
         orig = __float_as_uint(B.w);
         t = isect_sphere(make_float4(c.x, c.y, c.z, A.w), ro, rd, tmin);
       } else if (MESH) {
-        float4 a = sc.tri[3 * p], b = sc.tri[3 * p + 1], c = sc.tri[3 * p + 2];
+        float4 a = gp(sc.tri)[3 * p], b = gp(sc.tri)[3 * p + 1], c = gp(sc.tri)[3 * p + 2];
         float b1, b2;
         if (!tri_test(tr, ro, mk3(a), mk3(b), mk3(c), t, b1, b2)) t = FINF;
         orig = __float_as_uint(a.w);
@@ -424,11 +432,11 @@ struct Tracer {
       if (!(t > tmin)) continue;
       bool take = t < h.t;
       if (!take && t == h.t && h.pos >= 0) {
-        if (SPH && kind == PT_GEOM_SPHERES) orig = sc.sph_idx[p];
+        if (SPH && kind == PT_GEOM_SPHERES) orig = gp(sc.sph_idx)[p];
         take = wins_tie(sc, (int)orig);
       }
       if (take) {
-        if (SPH && kind == PT_GEOM_SPHERES && orig == 0xFFFFFFFFu) orig = sc.sph_idx[p];
+        if (SPH && kind == PT_GEOM_SPHERES && orig == 0xFFFFFFFFu) orig = gp(sc.sph_idx)[p];
         h.t = t;
         h.prim = (int)orig;
         h.pos = cur;

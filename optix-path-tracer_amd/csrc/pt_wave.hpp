@@ -338,7 +338,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
           }
         } else {
           int mat = hit_material(sc, pos, prim);
-          const DevMaterial& M = sc.mats[mat];
+          const DevMaterial& M = gp(sc.mats)[mat];
           bool need_uv = tex_needs_uv(sc, M.tex0) || (M.type == PT_MAT_ASHIKHMIN_SHIRLEY && tex_needs_uv(sc, M.tex1));
           const float tm = (EXT && sc.mov_instances) ? P.ptime[dw & SLOT_MASK] : 0.f;
           HitRec r = hit_record<KINDS, EXT>(sc, pos, prim, hit.x, mk3(o4), d, need_uv, tm);
@@ -382,7 +382,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
             if (nl > 0) {
               int index = ((int)(rnd(seed) * nl)) % nl;
               if (!(is_light && nl == 1)) {
-                const DevLight& Lt = lights[index];
+                const DevLight& Lt = gp(lights)[index];
                 const bool env = (FEAT & SH_ENV) && Lt.type == PT_LIGHT_ENV;
                 v3 Wi = env ? env_sample(sc, seed) : light_sample(Lt, r.P, seed);
                 float lightPDF = env ? env_pdf(sc, Wi) : light_pdf(Lt, r.P, Wi);
@@ -413,7 +413,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
                   const v3 emission = env ? env_radiance(sc, Wi) : light_emission(Lt);
                   bool occluded = false;
                   if (sh.pos >= 0)
-                    occluded = env || !(sc.mats[hit_material(sc, sh.pos, sh.prim)].type == PT_MAT_DIFFUSE_LIGHT &&
+                    occluded = env || !(gp(sc.mats)[hit_material(sc, sh.pos, sh.prim)].type == PT_MAT_DIFFUSE_LIGHT &&
                                         (iso || dot(r.N, Wi) > 0.f));
                   sig = sig_mix(sig, occluded ? 0xA5A5A5A5u : 0x5A5A5A5Au);
                   if (!occluded) {
