@@ -288,16 +288,39 @@ int grid_for(uint64_t n) {
   return (int)std::max<uint64_t>(1, std::min<uint64_t>((n + BLOCK - 1) / BLOCK, cap));
 }
 
+// Camera paths per wave of a batch of n paths (64: the dense set).  Below 2^18
+// paths full waves leave SIMDs idle while each wave goes through the different
+// nodes, leaves and materials of its 64 paths one after another; spread over
+// the 4096 waves the chip holds of the last-bounces launch, a wave has as few
+// as its share, and at least 2.  One frame and
+// its display, 64 against n / 4096 lanes: Cornell box 4 k paths 352 -> 283
+// us, 21 k 387 -> 331 us; spheres 10 k 423 -> 295 us; mesh scene 11 k 976 ->
+// 670 us, 130 k 1.46 -> 1.35 ms; next-week scene 10 k 2.02 -> 1.32 ms; from
+// 250 k on no difference.
+uint32_t lanes_for(uint64_t n) {
+  return n < (1u << 18) ? (uint32_t)std::min<uint64_t>(64, std::max<uint64_t>(2, (n + 4095) / 4096)) : 64u;
+}
+// blocks of a batch of n paths, `lanes` of them per wave
+int grid_of(uint64_t n, uint32_t lanes) {
+  return lanes == 64u ? grid_for(n) : (int)((n + lanes * (uint64_t)WAVES - 1) / (lanes * (uint64_t)WAVES));
+}
+
 // First bounce of the one launch that runs all the bounces left (SH_TAIL),
-// for a batch of n paths.  Its waves trace lock-step and unsorted, so it pays
-// from where a wave holds few paths: measured with 1, 2, 3, 4, 6 and 8 (and a
-// launch per kernel and bounce), 4 k paths of the Cornell box 339, 367, 389,
-// 401, 420, 458 (526) us; 1.0 M of the next-week scene 5.7, 4.9, 4.1, 3.9,
-// 4.4, 4.7 (10.5) ms; 1.7 M of the sphere scene 1.8, 1.8, 1.9, 2.0, 2.3, 2.5
-// (4.3) ms; 2.1 M of the mesh scene 4.2, 4.0, 4.6, 4.9, 5.4, 5.7 (6.0) ms;
-// 134 M of 16 scenes 70.7, 66.4, 67.0, 67.8, 67.6, 67.2 (70.0) ms; 199 M of
-// the mesh scene 85.1, 76.0, 74.6, 72.5, 71.9, 72.5 (73.3) ms.
-uint32_t tail_depth(uint64_t n) { return n < (1u << 18) ? 1u : n < (1u << 23) ? 3u : 4u; }
+// for a batch of n paths.  Its waves trace lock-step and unsorted, so large
+// sorted batches enter it where a wave holds few paths; unsorted ones and
+// those below 2^23 paths after the camera rays; media, boxes and procedural
+// textures (ext), whose materials diverge most, later.  Measured from bounce
+// 1, 2, 3, 4, 5, 6 on: 1.7 M paths of the sphere scene 1.57, 1.65, 1.71, 1.80,
+// 1.95, 2.09 ms; 2.1 M of the mesh scene 3.29, 3.41, 3.86, 4.16, 4.43, 4.63
+// ms; 1.0 M of the next-week scene (ext) 4.95, 4.25, 3.58, 3.40, 3.60, 3.69
+// ms; 16.8 M of the Cornell box (unsorted) 9.79, 9.93, 10.00, 10.13, 10.16,
+// 10.21 ms; 199 M of the mesh scene 71.7, 63.8, 61.6, 59.8, 59.9, 59.5 ms;
+// 134 M of 16 scenes 58.3, 56.6, 57.1, 57.7, 56.4, 57.8 ms.  With a launch per
+// kernel and bounce throughout these were 4.3, 6.0, 10.5, 10.4, 73 and 70 ms.
+uint32_t tail_depth(uint64_t n, bool sorted, bool ext) {
+  if (n < (1u << 18)) return 1u;
+  return ext || (sorted && n >= (1u << 23)) ? 4u : 1u;
+}
 
 // an odd stride near 0.618 n that is coprime to n (a full-period
 // multiplicative order of 0..n-1)
@@ -1263,7 +1286,10 @@ pt_status pt_render(pt_context* c, const pt_render_params* rp, uint32_t frame_be
   if (use_cache && !c->cache_ready) return fail(c, PT_ERR_STATE, "PT_FLAG_RADIANCE_CACHE needs pt_cache_init");
   if (use_cache && (c->dsc.ext_instances != 0 || (c->mat_types >> PT_MAT_ISOTROPIC) != 0))
     return fail(c, PT_ERR_UNSUPPORTED, "the radiance cache does not take volumes, isotropic or normal-shader materials");
-  pt_status ps = ensure_paths(c, (uint64_t)fpb * WH);
+  auto lanes_of = [&](uint64_t n) { return use_cache ? 64u : lanes_for(n); };
+  const uint64_t full = (uint64_t)fpb * WH;
+  auto positions = [&](uint64_t n) { return std::max<uint64_t>(n, (uint64_t)grid_of(n, lanes_of(n)) * WAVES * lanes_of(n)); };
+  pt_status ps = ensure_paths(c, positions(full));
   if (ps == PT_OK) ps = ensure_spill(c);
   if (ps != PT_OK) return ps;
   if (use_cache) {
@@ -1305,7 +1331,7 @@ pt_status pt_render(pt_context* c, const pt_render_params* rp, uint32_t frame_be
     int in = 0, out = 1;
     // with the radiance cache: not before the queries are asked, and not in
     // sorted batches (the sort's order is that of the training records)
-    uint32_t tail = tail_depth(nslots);
+    uint32_t tail = tail_depth(nslots, sort, c->dsc.ext_instances != 0 || (c->mat_types >> PT_MAT_ISOTROPIC) != 0);
     if (rc.flags & PT_FLAG_RADIANCE_CACHE) {
       if (rc.cache.query_depth < rp->max_depth) tail = std::max(tail, rc.cache.query_depth + 1);
       if (sort) tail = 0xFFFFFFFFu;
@@ -1348,7 +1374,8 @@ pt_status pt_render(pt_context* c, const pt_render_params* rp, uint32_t frame_be
     rc.frame0 = frame_begin + f0;
     // a held batch asks nothing (no path reaches this query depth)
     if (use_cache) rc.cache.query_depth = c->cache_hold ? 0xFFFFFFFFu : c->cache_query_depth;
-    const int grid = grid_for(nslots);
+    P.row = lanes_of(nslots);
+    const int grid = grid_of(nslots, P.row);
     if (use_graph && nf == fpb) {
       // full batches replay a graph captured once for this launch state;
       // the batch's first frame comes from frame_dev, advanced in-graph
@@ -1900,7 +1927,10 @@ pt_status render_batch_shaped(pt_context* const* ctxs, const pt_render_params* p
     HIPCHK(B, hipMemcpy(B->d_item_frame, frame.data(), nitems * 4, hipMemcpyHostToDevice));
   }
   if (max_slots) {
-    pt_status ps = ensure_paths(B, max_slots);
+    uint64_t need = max_slots;
+    for (uint32_t k : bslots)
+      if (k) need = std::max<uint64_t>(need, (uint64_t)grid_of(k, lanes_for(k)) * WAVES * lanes_for(k));
+    pt_status ps = ensure_paths(B, need);
     if (ps == PT_OK) ps = ensure_spill(B);
     if (ps != PT_OK) return ps;
   }
@@ -1940,12 +1970,13 @@ pt_status render_batch_shaped(pt_context* const* ctxs, const pt_render_params* p
       const uint32_t nslots = bslots[b];
       const size_t k0 = first[b], k1 = first[b + 1];
       if (nslots == 0) continue;
-      const int grid = grid_for(nslots);
+      P.row = lanes_for(nslots);
+      const int grid = grid_of(nslots, P.row);
       // the depth-0 closest-hit launch starts the sub-batch's camera paths
       const BatchStart bs{B->d_rcs, B->d_item_off + k0, B->d_item_scene + k0, B->d_item_frame + k0,
                           (uint32_t)(k1 - k0)};
       int in = 0, o = 1;
-      const uint32_t tail = (count_trav || (params[0].flags & PT_FLAG_DIRECT)) ? 0xFFFFFFFFu : tail_depth(nslots);
+      const uint32_t tail = (count_trav || (params[0].flags & PT_FLAG_DIRECT)) ? 0xFFFFFFFFu : tail_depth(nslots, sort, ext);
       for (uint32_t depth = 0; depth < max_depth; depth++) {
         if (depth == tail) {
           hipEvent_t a = kernel_events ? mark() : nullptr;

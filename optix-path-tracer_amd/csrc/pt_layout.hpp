@@ -197,6 +197,8 @@ struct DevCamera {
 // survivors (never more than its inputs) into its own segment of the output
 // set, so the hot loop takes no global atomic.  A dense set of n positions
 // is the case n_w = (positions of the segment below n).
+// A small batch puts fewer than 64 paths in a wave: rows of DevPaths::row
+// positions instead of 64 (one row per wave then holds them all).
 constexpr uint32_t SLOT_MASK = 0x3FFFFFFFu;
 constexpr uint32_t TRAIN_BIT = 1u << 30;  // radiance-cache training path
 constexpr uint32_t SPEC_BIT = 1u << 31;   // last bounce was specular
@@ -209,6 +211,7 @@ struct PathState {
 };
 
 struct DevPaths {
+  uint32_t row;         // positions per wave and row of a segment (64, or fewer in small batches)
   PathState st[3];      // [0], [1] ping-pong, [2] material-sorted copy
   float4* hit;          // per active path of the input set: (t, instance position, prim, instance id)
   float4* hit_sorted;

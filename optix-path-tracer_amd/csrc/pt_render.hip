@@ -210,9 +210,9 @@ PTD PathStart start_path(const DevPaths& P, const RenderConsts& rc, uint32_t p, 
   P.result[s] = make_float4(0.f, 0.f, 0.f, __uint_as_float(rc.max_depth));
   return PathStart{o4, d4, tm};
 }
-PTD void reset_segments(const DevPaths& P, uint32_t nslots, const Seg& g) {
+PTD void reset_segments(const DevPaths& P, uint32_t n, const Seg& g) {
   if (__lane_id() == 0) {
-    P.seg[g.w] = dense_count(nslots, g);
+    P.seg[g.w] = n;
     P.tseg[g.w] = 0u;
     P.qseg[g.w] = 0u;
   }
@@ -255,13 +255,13 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(extend_wa
   constexpr int NS = extend_stk<KINDS>();
   __shared__ uint2 s_stk[NS * BLOCK];
   StackT<NS> st = make_stack<NS>(s_stk, spill, P.counters + CTR_STACK_OVERFLOW);
-  const Seg g = my_seg();
+  const Seg g = my_seg(P);
   constexpr bool starts = START;
   uint32_t n;
   if (starts) {
     if (!MULTI && rc.frame_dev) rc.frame0 = *rc.frame_dev;  // replayed graphs take the batch's frame from memory
     n = dense_count(nstart, g);
-    reset_segments(P, nstart, g);
+    reset_segments(P, n, g);
   } else {
     n = seg_count(P, in, g);
   }
@@ -459,7 +459,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_sort_scan(DevPaths P, uint32_t
 // Move path state and hit into material-bucket order (state set 2, a dense
 // set): each wave writes its bucket-b paths from its scanned base on.
 __global__ __launch_bounds__(BLOCK) void k_sort_scatter(DevPaths P, int in) {
-  const Seg g = my_seg();
+  const Seg g = my_seg(P);
   const uint32_t n = seg_count(P, in, g);
   const PathState S = P.st[in], D = P.st[2];
   uint32_t cur[8];
@@ -489,7 +489,7 @@ __global__ __launch_bounds__(BLOCK) void k_sort_scatter(DevPaths P, int in) {
 // Paths alive after the last bounce end with color() = 0 (raygen.cu:121-122);
 // only their signature is recorded.
 __global__ __launch_bounds__(BLOCK) void k_exhausted(DevPaths P, int in, uint64_t* stats) {
-  const Seg g = my_seg();
+  const Seg g = my_seg(P);
   const uint32_t n = seg_count(P, in, g);
   const PathState S = P.st[in];
   if (__lane_id() == 0) stat_add(stats, g, STAT_EXHAUSTED, n);
@@ -611,7 +611,7 @@ __global__ __launch_bounds__(BLOCK) void k_cache_gather(DevPaths P, int which, u
 // The queries' answers: result += T * cache_radiance(y) per channel, over
 // each wave's query segment (same grid as the batch).
 __global__ __launch_bounds__(BLOCK) void k_cache_apply(DevPaths P) {
-  const Seg g = my_seg();
+  const Seg g = my_seg(P);
   const uint32_t n = uniform(P.qseg[g.w]);
   for (uint32_t j = __lane_id(); j < n; j += 64) {
     const uint32_t i = g.pos(j);
@@ -693,7 +693,7 @@ __global__ __launch_bounds__(BLOCK) void k_accumulate(DevPaths P, RenderConsts r
     accum[o + 2] = a2;
   }
   for (int d = 32; d >= 1; d >>= 1) nans += __shfl_xor(nans, d);
-  if (__lane_id() == 0) stat_add(stats, my_seg(), STAT_NAN, nans);
+  if (__lane_id() == 0) stat_add(stats, my_seg(P), STAT_NAN, nans);
 }
 
 // raygen.cu:136-146 make_Color on the FP64 accumulation

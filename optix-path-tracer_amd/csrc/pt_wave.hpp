@@ -13,19 +13,20 @@ PTD uint32_t lane_rank(uint64_t mask) {
 }
 // This wave's segment of a path set (layout in pt_layout.hpp).
 struct Seg {
-  uint32_t stride;  // G * BLOCK
-  uint32_t base;    // b * BLOCK + v * 64
+  uint32_t stride;  // waves of the grid * row
+  uint32_t base;    // w * row
   uint32_t w;       // wave index in the grid
+  uint32_t row;     // with fewer than 64 the segment is one row
   PTD uint32_t pos(uint32_t j) const { return (j >> 6) * stride + base + (j & 63u); }
 };
-PTD Seg my_seg() {
-  const uint32_t v = threadIdx.x >> 6;
-  return Seg{gridDim.x * BLOCK, blockIdx.x * BLOCK + v * 64u, blockIdx.x * WAVES + v};
+PTD Seg my_seg(const DevPaths& P) {
+  const uint32_t w = blockIdx.x * WAVES + (threadIdx.x >> 6);
+  return Seg{gridDim.x * WAVES * P.row, w * P.row, w, P.row};
 }
 // positions of the segment below n: the segment count of a dense set
 PTD uint32_t dense_count(uint32_t n, const Seg& g) {
   const uint32_t full = n / g.stride, r = n - full * g.stride;
-  return full * 64u + (r > g.base ? min(r - g.base, 64u) : 0u);
+  return full * g.row + (r > g.base ? min(r - g.base, g.row) : 0u);
 }
 PTD uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 // live paths of this wave's segment of state set `set`
@@ -262,7 +263,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
   // spills; with the stack, 36 KB per block keeps 4 blocks of 4 waves per CU)
   __shared__ float s_keep[12 * BLOCK];
   StackT<STK_LDS_SHADE> st = make_stack<STK_LDS_SHADE>(s_stk, spill, P.counters + CTR_STACK_OVERFLOW);
-  const Seg g = my_seg();
+  const Seg g = my_seg(P);
   uint32_t depth = depth0;
   uint32_t n = seg_count(P, src, g);
   PathState S = P.st[src], D = P.st[out];

@@ -109,10 +109,12 @@ def test_facade_launch_loop_equals_render(tmp_path, scene, cfg, W, H, frames):
 
 
 # depths around the bounce where one launch takes over the rest of a batch
-# (1 or 3 at these sizes), a path count below one wave, and 2^18 + 1 paths
+# (1, or 4 in the extended scenes from 2^18 paths on), a path count below one
+# wave, and image sizes around 2^18 paths, where waves start with fewer lanes
 @pytest.mark.parametrize("cfg,W,H,frames,depths", [
     (ptamd.PT_SCENE_CORNELL, 7, 5, 1, (1, 2, 3)), (ptamd.PT_SCENE_CORNELL, 96, 64, 2, (1, 2, 16)),
-    (ptamd.PT_SCENE_RANDOM_SPHERES, 513, 511, 1, (1, 3, 4, 50)), (ptamd.PT_SCENE_MESHES, 61, 47, 3, (2, 12)),
+    (ptamd.PT_SCENE_RANDOM_SPHERES, 513, 511, 1, (1, 50)), (ptamd.PT_SCENE_CORNELL, 512, 512, 1, (1, 2, 5)),
+    (ptamd.PT_SCENE_RANDOM_SPHERES, 91, 45, 1, (2, 50)), (ptamd.PT_SCENE_NEXT_WEEK, 513, 512, 1, (4, 5, 9)), (ptamd.PT_SCENE_MESHES, 61, 47, 3, (2, 12)),
     (ptamd.PT_SCENE_NEXT_WEEK, 61, 47, 2, (2, 50)), (ptamd.PT_SCENE_MOVING_SPHERES, 61, 47, 2, (3, 50))])
 def test_last_bounces_in_one_launch_are_bit_identical(ctx, cfg, W, H, frames, depths):
     sc = setup(ctx, cfg, W, H, 3 if cfg == ptamd.PT_SCENE_MESHES else 0)
