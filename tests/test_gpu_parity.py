@@ -798,6 +798,25 @@ def awkward_rays(n, lo, hi, seed):
     return rays
 
 
+def test_host_queries_across_the_kept_buffer(ctx):
+    """Host-array queries keep a device buffer of up to 64 MiB: calls that
+    grow it, fit it, exceed it (1.5 M rays) and fit it again answer alike."""
+    sc = ptamd.Scene(ptamd.PT_SCENE_CORNELL, 64, 64)
+    ctx.set_scene(sc.desc)
+    ctx.build_accel()
+    rays = random_rays(1_500_000, 0.0, 555.0, 5)
+    say("[gpu] host queries: 7, 1.5 M and 2 x 0.75 M rays")
+    first = ctx.trace_closest(rays[:7])
+    whole, occ = ctx.trace_closest(rays), ctx.trace_occluded(rays)
+    half = len(rays) // 2
+    parts = np.concatenate([ctx.trace_closest(rays[:half]), ctx.trace_closest(rays[half:])])
+    assert np.array_equal(whole.view(np.uint8), parts.view(np.uint8))
+    assert np.array_equal(whole[:7].view(np.uint8), first.view(np.uint8))
+    assert np.array_equal(occ, np.concatenate([ctx.trace_occluded(rays[:half]), ctx.trace_occluded(rays[half:])]))
+    hits, counts = ctx.trace_closest(rays[half:], counted=True)
+    assert np.array_equal(hits.view(np.uint8), parts[half:].view(np.uint8)) and counts[:, 0].min() >= 1
+
+
 # The kernels that count use the exact slab test, the others a conservative
 # one with fused multiply-adds: they visit the same leaves and at times one
 # more, so their hit is never behind the exact test's, or behind it in a tie.
