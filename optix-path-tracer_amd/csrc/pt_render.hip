@@ -355,7 +355,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(extend_wa
         }
         o = ps.o;
         d = ps.d;
-        if (EXT && sc0.mov_instances) tm = ps.tm;
+        if (EXT && (MULTI || sc0.mov_instances)) tm = ps.tm;  // a batch's scenes differ: sc0 is the first one's
       } else {
         o = S.o[i];
         d = S.d[i];

@@ -108,6 +108,22 @@ def test_batch_with_media_and_moving_spheres_equals_single_renders():
             ctx.close()
 
 
+def test_batch_moving_spheres_after_a_still_scene():
+    """Whether camera rays carry their time is the path's own scene's
+    matter: moving spheres behind a scene that has none keep their blur."""
+    made = [make(ptamd.PT_SCENE_CORNELL, 32, 32), make(ptamd.PT_SCENE_MOVING_SPHERES, 40, 27)]
+    try:
+        alone = [single(sc, ctx, 2) for sc, ctx in made]
+        say("[gpu] batch: cornell, moving spheres")
+        ptamd.render_batch([c for _, c in made], [s.render_params() for s, _ in made], [2, 2])
+        for (sc, ctx), (acc, _, _) in zip(made, alone):
+            got, _ = ctx.read_accum(sc.info.width, sc.info.height)
+            assert np.array_equal(got, acc)
+    finally:
+        for _, ctx in made:
+            ctx.close()
+
+
 def test_batch_graph_replay_is_bit_identical(scenes):
     """PT_FLAG_GRAPH in params[0]: the whole batch is captured once and
     replayed; every replay (with other renders of the same contexts in
