@@ -246,9 +246,11 @@ PTD bool scatter_and_roulette(const Surface& f, v3 Wo, v3 N, uint32_t& seed, uin
 // material sort, whatever the number of paths; a wave's own chain of rays
 // is shorter than the sum of the batch's longest ones.  The paths' results
 // do not depend on the order they are traced in: images are the same bit
-// for bit.  Against a launch per kernel and bounce: 64x64 Cornell tile 526
-// -> 339 us, random spheres 4.29 -> 1.9 ms, next-week scene 10.5 -> 4.1 ms,
-// one 1080p frame of the mesh scene 6.0 -> 4.6 ms.
+// for bit.  Against a launch per kernel and bounce, the kernels otherwise as
+// they were then: 64x64 Cornell tile 526 -> 339 us, random spheres 4.29 ->
+// 1.9 ms, next-week scene 10.5 -> 4.1 ms, one 1080p frame of the mesh scene
+// 6.0 -> 4.6 ms (257 us, 1.4, 3.4 and 3.4 ms with the traversal and the
+// spread of small batches of today).
 constexpr int SH_COUNT = 1, SH_CACHE = 2, SH_ENV = 4, SH_MULTI = 8, SH_EXT = 16, SH_TAIL = 32;
 template <int MS, int FEAT, int KINDS = KIND_ALL>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_shade(
