@@ -378,9 +378,9 @@ pt_status pt_render(struct pt_context* ctx, const pt_render_params* params,
 /* No counterpart in the reference (it renders one scene per OptiX context;
  * this replaces its per-scene launch loop, main.cpp:26-39,264-265):
  * frames [0, frame_counts[i]) of every ctxs[i], i < n <= 256, in one
- * wavefront.  The (scene, frame) work items are cut into sub-batches of at
- * most the automatic batch size of ctxs[0] (see frames_per_batch); within a
- * sub-batch all paths share one path pool and
+ * wavefront.  The (scene, frame) work items are cut into even sub-batches of
+ * about 2^27 paths, at most the automatic batch size of ctxs[0] (see
+ * frames_per_batch); within a sub-batch all paths share one path pool and
  * one launch per kernel and bounce, so many small or uneven scenes fill the
  * GPU together.  Every context needs a built scene and a camera, all on one
  * device; ctxs[0] runs the batch.  Each context's accumulation restarts at

@@ -2108,16 +2108,35 @@ pt_status render_batch_shaped(pt_context* const* ctxs, const pt_render_params* p
 
 extern "C" {
 
+// Paths per sub-batch of a batch of scenes whose shape is not tuned: even
+// parts nearest to 2^27 paths (a frame more, since frames are not split).
+// Each launch is a latency-bound tail after its bulk, so parts must be large,
+// but scenes in flight together share the caches.  Parts of at most 2^24,
+// 2^25, 2^26, 2^27 and 2^29 paths: all 64 scenes of the mixed batch (497 M
+// paths) 251, 220, 217, 203, 218 ms; its 32 sphere scenes (238 M) 109, 104,
+// 104, 97, 98 ms; its 32 mesh scenes (259 M) 142, 119, 109, 103, 104 ms; 16 of
+// them (134 M) 66, 59, 56, 54, 55 ms.
+static uint64_t batch_paths(const pt_render_params* params, const uint32_t* frame_counts, uint32_t n) {
+  uint64_t total = 0, frame = 0;
+  for (uint32_t i = 0; i < n; i++) {
+    const uint64_t WH = (uint64_t)params[i].width * params[i].height;
+    total += WH * frame_counts[i];
+    frame = std::max(frame, WH);
+  }
+  const uint64_t parts = std::max<uint64_t>(1, (total + (1ull << 26)) >> 27);
+  return total / parts + frame;
+}
+
 pt_status pt_render_batch(pt_context* const* ctxs, const pt_render_params* params, const uint32_t* frame_counts,
                           uint32_t n, pt_render_stats* out) {
   if (!ctxs || !params || !frame_counts || n == 0 || !ctxs[0]) return PT_ERR_INVALID_ARG;
   pt_context* B = ctxs[0];
   if (n > 256) return fail(B, PT_ERR_INVALID_ARG, "at most 256 scenes per batch");
   // the shape: the one pt_autotune_batch picked for this composition when
-  // params[0] asks for it, else ~16 Mi paths per sub-batch and
+  // params[0] asks for it, else even sub-batches of about 2^27 paths and
   // params[0]'s material-sort and graph flags
   BatchShape shape;
-  shape.paths = B->paths_target;
+  shape.paths = std::min<uint64_t>(B->paths_target, batch_paths(params, frame_counts, n));
   const uint32_t f0 = params[0].flags;
   shape.sort = (f0 & PT_FLAG_MATERIAL_SORT) != 0;
   shape.graph = (f0 & PT_FLAG_GRAPH) != 0;

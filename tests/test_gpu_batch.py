@@ -226,6 +226,31 @@ def test_batch_split_across_path_pools(scenes):
         big.close()
 
 
+def test_large_batch_in_even_parts():
+    """Above 1.5 x 2^27 paths a batch runs in even parts of about 2^27; a
+    part's edge falls between two frames of the middle scene."""
+    made = [make(ptamd.PT_SCENE_RANDOM_SPHERES, 1000, 667), make(ptamd.PT_SCENE_CORNELL, 1024, 1024),
+            make(ptamd.PT_SCENE_CORNELL, 33, 21)]
+    try:
+        frames = [60, 160, 3]
+        assert sum(sc.info.width * sc.info.height * f for (sc, _), f in zip(made, frames)) > 3 << 26
+        alone = []
+        for (sc, ctx), f in zip(made, frames):
+            say(f"[gpu] single render {sc.info.width}x{sc.info.height} x {f}")
+            alone.append(single(sc, ctx, f))
+        say("[gpu] batch in two parts")
+        st = ptamd.render_batch([c for _, c in made], [s.render_params() for s, _ in made], frames)
+        for (sc, ctx), (acc, n, _), f in zip(made, alone, frames):
+            got, m = ctx.read_accum(sc.info.width, sc.info.height)
+            assert m == n == f
+            assert np.array_equal(got, acc)
+        assert st.extension_rays == sum(a[2].extension_rays for a in alone)
+        assert st.shadow_rays == sum(a[2].shadow_rays for a in alone)
+    finally:
+        for _, ctx in made:
+            ctx.close()
+
+
 def test_batch_rejects_bad_input(scenes):
     sc, ctx = scenes[0]
     p = sc.render_params()
