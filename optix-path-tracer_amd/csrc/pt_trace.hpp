@@ -181,23 +181,27 @@ struct Tracer {
 
   // Constants of node_fast for the ray (ro, rd): the reciprocal of each
   // component, at most 2^100 in magnitude (a zero component gives no inf - inf
-  // with the scene's planes), and the two offsets.  A component that is NaN,
-  // infinite or above 2^100 gives NaN distances, which the minima and maxima
+  // with the scene's planes), and the two offsets.  Where that bound cuts the
+  // reciprocal the planes move out by another 2^80 (1e-6 of a length unit): a
+  // ray that runs within a slab never leaves it, also in the plane of a face at
+  // 0, where the plane's distance and its margin are both zero.  A component
+  // that is NaN or infinite gives NaN distances, which the minima and maxima
   // pass over: that axis then rejects nothing.
-  PTD static float bound_rcp(float x) {
-    float m = fabsf(__builtin_amdgcn_rcpf(x));
-    m = m > 0x1p100f ? 0x1p100f : m;
-    m = m < 0x1p-100f ? __builtin_nanf("") : m;
-    return copysignf(m, x);
+  PTD static float bound_rcp(float x, float& room) {
+    const float r = __builtin_amdgcn_rcpf(x);
+    room = fabsf(r) > 0x1p100f ? 0x1p80f : 0.f;
+    return __builtin_fmaf(x, 0.f, __builtin_amdgcn_fmed3f(r, -0x1p100f, 0x1p100f));
   }
   PTD void setup() {
     if (KEEP_INV) rinv = mk3(1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z);
     if (FAST) fast_setup();
   }
   PTD void fast_setup() {
-    finv = mk3(bound_rcp(rd.x), bound_rcp(rd.y), bound_rcp(rd.z));
+    v3 room;
+    finv = mk3(bound_rcp(rd.x, room.x), bound_rcp(rd.y, room.y), bound_rcp(rd.z, room.z));
     const v3 a = mk3(ro.x * finv.x, ro.y * finv.y, ro.z * finv.z);
-    const v3 e = mk3(fabsf(a.x) * 0x1p-21f, fabsf(a.y) * 0x1p-21f, fabsf(a.z) * 0x1p-21f);
+    const v3 e = mk3(__builtin_fmaf(fabsf(a.x), 0x1p-21f, room.x), __builtin_fmaf(fabsf(a.y), 0x1p-21f, room.y),
+                     __builtin_fmaf(fabsf(a.z), 0x1p-21f, room.z));
     nb = mk3(-a.x - e.x, -a.y - e.y, -a.z - e.z);
     fb = mk3(e.x - a.x, e.y - a.y, e.z - a.z);
     sx = finv.x < 0.f ? 16u : 0u;

@@ -1,0 +1,91 @@
+"""Rays that meet the conservative node test (the kernels that do not count)
+at its edges, against the exact one (the kernels that count)."""
+import sys
+
+import numpy as np
+import pytest
+
+import ptamd
+from helpers import PyScene
+
+pytestmark = pytest.mark.gpu
+
+
+def say(msg):
+    print(msg, flush=True)
+    sys.stdout.flush()
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = ptamd.Context(0)
+    yield c
+    c.close()
+
+
+def same(a, b):
+    return (a["t"] == b["t"]) & (a["inst"] == b["inst"]) & (a["prim"] == b["prim"])
+
+
+def rays_of(org, d, tmin, tmax=np.inf):
+    r = np.zeros(len(org), ptamd.RAY_DTYPE)
+    r["org"], r["dir"], r["tmin"], r["tmax"] = org, d, tmin, tmax
+    return r
+
+
+def faces_at_zero():
+    """Boxes and rects with faces and edges in the planes x, y, z = 0."""
+    rng = np.random.default_rng(3)
+    s = PyScene()
+    m = s.lambert((0.5, 0.5, 0.5))
+    for q in range(96):
+        lo, hi = np.sort(rng.uniform(-8, 8, (2, 3)), axis=0)
+        axis = q % 3
+        lo[axis], hi[axis] = (0.0, abs(hi[axis]) + 0.1) if q % 2 else (-abs(lo[axis]) - 0.1, 0.0)
+        s.boxes.append((tuple(lo), tuple(hi), m))
+        a, b = np.sort(rng.uniform(-8, 8, (2, 2)), axis=1)
+        e = a if q % 4 < 2 else b
+        e[q % 2] = 0.0
+        e.sort()
+        s.rects.append((axis, 0, a[0], a[1], b[0], b[1], float(rng.uniform(-8, 8)), m))
+    s.instance(ptamd.PT_GEOM_BOXES, 0, 48)
+    s.instance(ptamd.PT_GEOM_RECTS, 0, 48)
+    for q in range(48, 96):
+        s.instance(ptamd.PT_GEOM_BOXES, q, 1)
+        s.instance(ptamd.PT_GEOM_RECTS, q, 1)
+    return s, m
+
+
+@pytest.mark.parametrize("mesh", [False, True])
+def test_rays_in_the_planes_of_faces(ctx, mesh):
+    """Directions with zero components from origins in a face's or an edge's
+    own plane at 0, where the rounding margins of the node test are zero: such
+    a ray runs along edges, which belong to the faces, and (octahedra) between
+    two triangles that both have the edge."""
+    rng = np.random.default_rng(4)
+    s, m = faces_at_zero()
+    if mesh:
+        v = np.float32([[2, 0, 0], [-2, 0, 0], [0, 2, 0], [0, -2, 0], [0, 0, 2], [0, 0, -2]])
+        f = np.uint32([[a, b, c] for a in (0, 1) for b in (2, 3) for c in (4, 5)])
+        for q in range(8):  # a mesh each
+            s.meshes.append((v * np.float32(0.2 + 0.3 * q), f, None, None, m))
+            s.instance(ptamd.PT_GEOM_MESH, q, 0)
+    n = 60000
+    k = np.arange(n)
+    org = rng.uniform(-9, 9, (n, 3))
+    d = rng.normal(size=(n, 3))
+    axis = rng.integers(0, 3, n)
+    org[k, axis] = rng.choice([0.0, -0.0, 1e-30, -1e-30], n)
+    d[k, axis] = rng.choice([0.0, -0.0], n)
+    second = k[k % 3 == 0]
+    d[second, (axis[second] + 1) % 3] = 0.0
+    rays = rays_of(org, d, 1e-3)
+    desc = s.desc()
+    say(f"[gpu] rays in the planes of faces, meshes {mesh}: {n} rays")
+    ctx.set_scene(desc)
+    ctx.build_accel()
+    a = ctx.trace_closest(rays)
+    b, _ = ctx.trace_closest(rays, counted=True)
+    differ = ~same(a, b)
+    assert (b["inst"] >= 0).mean() > 0.3
+    assert not differ.any(), f"{differ.sum()} of {n} rays"
