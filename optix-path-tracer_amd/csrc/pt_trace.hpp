@@ -4,9 +4,10 @@
 // One ray per lane.  The traversal stack keeps its top entries in LDS (one
 // column per lane, bank-conflict free; how many is the kernel's choice) and
 // spills deeper entries to a per-thread slice of HBM.  Children are visited
-// nearest first by entry distance (ties by slot); popped entries farther
-// than the current hit are skipped.  Candidates win on smaller t, ties on the smaller
-// (instance, primitive) key, so the result does not depend on visit order.
+// nearest first by entry distance; popped entries farther than the current hit
+// are skipped (with node_fast's margin where its distances are compared).
+// Candidates win on smaller t, ties on the smaller (instance, primitive) key,
+// so the result does not depend on visit order.
 #pragma once
 
 #include "pt_device.hpp"
@@ -221,7 +222,10 @@ struct Tracer {
   // every plane outward by 8 u |o inv| and the far distance grows by 32 u of
   // itself, which also covers the exact test's own rounding: the children
   // taken are those of the exact test, and now and then one more, whose
-  // primitives cannot win a closer hit.  Empty slots (inf planes) always
+  // primitives cannot win a closer hit.  An entry on the stack is compared
+  // with the hit found meanwhile: its distance may lie 6 u of itself above a
+  // primitive's in the same plane, so the hit's distance grows by the same
+  // 32 u there too (cull).  Empty slots (inf planes) always
   // fail, or, for a ray of NaNs, lead to a leaf of no primitives.
   //
   // Sorted by a network of five exchanges, reference and distance stored
@@ -294,6 +298,11 @@ struct Tracer {
       node_base = base;
   }
 
+  // an entry this far away holds nothing nearer than, or as near as, the hit
+  PTD bool cull(float etn) const {
+    return etn > (FAST ? __builtin_fmaf(fabsf(h.t), 0x1p-19f, h.t) : h.t);
+  }
+
   PTD bool at_node() const { return have && !(ref & LEAF_BIT); }
 
   // the entry in hand, from the stack when there is none; false: the ray is
@@ -312,7 +321,7 @@ struct Tracer {
       if (st.sp == 0) return false;
       float etn;
       st.pop(ref, etn);
-      have = !(etn > h.t);
+      have = !cull(etn);
     }
     return true;
   }

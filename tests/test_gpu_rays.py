@@ -1,12 +1,13 @@
 """Rays that meet the conservative node test (the kernels that do not count)
-at its edges, against the exact one (the kernels that count)."""
+at its edges, against the exact one (the kernels that count) and the oracle."""
 import sys
 
 import numpy as np
 import pytest
 
 import ptamd
-from helpers import PyScene
+import ptref
+from helpers import PyScene, icosphere
 
 pytestmark = pytest.mark.gpu
 
@@ -31,6 +32,56 @@ def rays_of(org, d, tmin, tmax=np.inf):
     r = np.zeros(len(org), ptamd.RAY_DTYPE)
     r["org"], r["dir"], r["tmin"], r["tmax"] = org, d, tmin, tmax
     return r
+
+
+# Overlapping rects in one plane k, as one group and as instances of their
+# own: every ray meets many hits at the same distance, and the smallest
+# (instance, primitive) wins, however the subtrees' entry distances round.
+# The padding of a flat box (1e-4) is less than the rounding of a distance
+# from k = 420 on.
+@pytest.mark.parametrize("k", [400.0, 555.0, 4000.0, 30000.0, 400000.0])
+@pytest.mark.parametrize("mesh", [False, True])
+def test_equal_distances_go_to_the_smallest_key(ctx, k, mesh):
+    rng = np.random.default_rng(int(k))
+    s = PyScene()
+    m = s.lambert((0.5, 0.5, 0.5))
+
+    def rect(axis):
+        a, b = np.sort(rng.uniform(-100, 100, (2, 2)), axis=1)
+        return (axis, 0, a[0], a[1], b[0], b[1], k, m)
+
+    s.rects = [rect(q % 3) for q in range(600)]
+    s.instance(ptamd.PT_GEOM_RECTS, 0, 300)
+    for q in range(300, 600):
+        s.instance(ptamd.PT_GEOM_RECTS, q, 1)
+    for q in rng.permutation(300)[:60]:  # duplicates of earlier rects
+        s.instance(ptamd.PT_GEOM_RECTS, 300 + int(q), 1)
+    if mesh:  # the kernels for scenes with meshes (lanes take rays one after another)
+        v, f = icosphere(2, 50.0, (-500.0, -500.0, -500.0))
+        s.meshes.append((v, f, None, None, m))
+        s.instance(ptamd.PT_GEOM_MESH, 0, 0)
+    desc = s.desc()
+    n = 60000
+    axis = np.arange(n) % 3
+    # origins at and near 0 on the facing axis, where the plane's distance
+    # takes all of its rounding from the reciprocal
+    org = rng.uniform(-60, 60, (n, 3))
+    near = rng.choice([0.0, 1e-3, 0.3, 1.0, 7.0], n) * rng.uniform(-1, 1, n)
+    org[np.arange(n), axis] = near
+    to = rng.uniform(-90, 90, (n, 3))
+    to[np.arange(n), axis] = k
+    rays = rays_of(org, (to - org) * rng.uniform(0.1, 3.0, (n, 1)), 1e-3)
+    say(f"[gpu] equal distances at {k}, meshes {mesh}: {n} rays")
+    ctx.set_scene(desc)
+    ctx.build_accel()
+    a = ctx.trace_closest(rays)
+    b, _ = ctx.trace_closest(rays, counted=True)
+    o = ptref.OracleScene(desc).trace(rays, brute=True)
+    assert (o["inst"] >= 0).mean() > 0.5
+    assert np.array_equal(a["t"], o["t"])
+    differ = ~same(a, o)
+    assert not differ.any(), f"{differ.sum()} of {n} rays"
+    assert same(b, o).all()
 
 
 def faces_at_zero():
