@@ -79,7 +79,7 @@ __global__ __launch_bounds__(BLOCK) void k_trace_closest(DevScene sc, const pt_r
                                                          uint2* spill, uint32_t* overflow) {
   __shared__ uint2 s_stk[STK_LDS * BLOCK];
   Stack st = make_stack(s_stk, spill, overflow);
-  Tracer<COUNT, EXT> tr;
+  Tracer<COUNT, EXT, KIND_ALL, false, false, true> tr;
   TraceCounts c;
   trace_queries<EXT, REFILL>(sc, rays, n, st, tr, c, [&](uint64_t i) {
     const HitOut& h = tr.h;
@@ -103,7 +103,7 @@ __global__ __launch_bounds__(BLOCK) void k_trace_occluded(DevScene sc, const pt_
                                                           uint32_t* overflow) {
   __shared__ uint2 s_stk[STK_LDS * BLOCK];
   Stack st = make_stack(s_stk, spill, overflow);
-  Tracer<COUNT, EXT> tr;
+  Tracer<COUNT, EXT, KIND_ALL, false, false, true> tr;
   TraceCounts c;
   trace_queries<EXT, REFILL>(sc, rays, n, st, tr, c, [&](uint64_t i) {
     const HitOut& h = tr.h;

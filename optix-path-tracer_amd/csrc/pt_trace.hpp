@@ -95,7 +95,10 @@ constexpr uint32_t TRIPS_MAX = 1u << 22;
 // kernels carry no trace of the early exit (a runtime-false flag still
 // changes their traversal loop's code and costs them about a tenth of
 // their time).
-template <bool COUNT, bool EXT = false, int KINDS = KIND_ALL, bool ANY = false, bool WIDE = false>
+//
+// QUERY: a caller's rays, whose directions may have any length (see
+// fast_setup).
+template <bool COUNT, bool EXT = false, int KINDS = KIND_ALL, bool ANY = false, bool WIDE = false, bool QUERY = false>
 struct Tracer {
   static constexpr bool SPH = (KINDS & 1) != 0, RECT = (KINDS & 2) != 0, BOX = (KINDS & 4) != 0,
                         MESH = (KINDS & 8) != 0;
@@ -111,6 +114,7 @@ struct Tracer {
   // far planes; byte offsets of the near planes in a node
   v3 finv, nb, fb;
   uint32_t sx, sy, sz;
+  float scale;  // QUERY: node distances are t * scale
   float tmin, time;
   uint32_t vseed;
   TriRay tr;
@@ -185,21 +189,43 @@ struct Tracer {
   // with the scene's planes), and the two offsets.  Where that bound cuts the
   // reciprocal the planes move out by another 2^80 (1e-6 of a length unit): a
   // ray that runs within a slab never leaves it, also in the plane of a face at
-  // 0, where the plane's distance and its margin are both zero.  A component
-  // that is NaN or infinite gives NaN distances, which the minima and maxima
-  // pass over: that axis then rejects nothing.
+  // 0, where the plane's distance and its margin are both zero.  An infinite
+  // component has distances 0, as in the exact test; a NaN one has NaN
+  // distances, which the minima and maxima pass over: that axis then rejects
+  // nothing.
+  //
+  // The bound holds for directions whose largest component lies between 2^-60
+  // and 2^100, as the renderer's do: its rays start with the camera's and
+  // instances' scales and are normalised or nearly so at each bounce.  QUERY
+  // brings directions outside 2^-40 .. 2^40 there by a power of two and keeps
+  // all node distances in that scale; a caller's shorter directions (below
+  // 1e-30) would otherwise lose the ratios of their components.
   PTD static float bound_rcp(float x, float& room) {
     const float r = __builtin_amdgcn_rcpf(x);
     room = fabsf(r) > 0x1p100f ? 0x1p80f : 0.f;
-    return __builtin_fmaf(x, 0.f, __builtin_amdgcn_fmed3f(r, -0x1p100f, 0x1p100f));
+    const float m = __builtin_amdgcn_fmed3f(r, -0x1p100f, 0x1p100f);
+    return x != x ? x : m;
   }
   PTD void setup() {
     if (KEEP_INV) rinv = mk3(1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z);
     if (FAST) fast_setup();
   }
   PTD void fast_setup() {
+    v3 u = rd;
+    if (QUERY) {
+      scale = 1.f;
+      const uint32_t m = __float_as_uint(fmaxf(fmaxf(fabsf(rd.x), fabsf(rd.y)), fabsf(rd.z)));
+      constexpr uint32_t LO = (127u - 40u) << 23, HI = (127u + 40u) << 23;
+      if (m - LO > HI - LO && m != 0u && m < 0x7F800000u) {
+        // the power of two of m, 2^-126 .. 2^126, and its reciprocal
+        const uint32_t e = min(max(m & 0x7F800000u, 0x00800000u), 0x7E800000u);
+        const float s = __uint_as_float(0x7F000000u - e);
+        scale = __uint_as_float(e);
+        u = mk3(rd.x * s, rd.y * s, rd.z * s);
+      }
+    }
     v3 room;
-    finv = mk3(bound_rcp(rd.x, room.x), bound_rcp(rd.y, room.y), bound_rcp(rd.z, room.z));
+    finv = mk3(bound_rcp(u.x, room.x), bound_rcp(u.y, room.y), bound_rcp(u.z, room.z));
     const v3 a = mk3(ro.x * finv.x, ro.y * finv.y, ro.z * finv.z);
     const v3 e = mk3(__builtin_fmaf(fabsf(a.x), 0x1p-21f, room.x), __builtin_fmaf(fabsf(a.y), 0x1p-21f, room.y),
                      __builtin_fmaf(fabsf(a.z), 0x1p-21f, room.z));
@@ -209,6 +235,8 @@ struct Tracer {
     sy = finv.y < 0.f ? 48u : 32u;
     sz = finv.z < 0.f ? 80u : 64u;
   }
+  // a distance along the ray as node_fast counts it
+  PTD float node_dist(float t) const { return QUERY ? t * scale : t; }
 
   // One internal node: the children the ray may enter, the nearest taken
   // next and the others on the stack, second nearest on top.
@@ -262,11 +290,12 @@ struct Tracer {
       nz = ld(sz); fz = ld(sz ^ 16u);
       cr = *reinterpret_cast<const u4*>(b + (p | 96u));
     }
+    const float lo = node_dist(tmin), hi = node_dist(h.t);
     auto slab = [&](float ax, float bx, float ay, float by, float az, float bz) {
       const float tn = fmaxf(fmaxf(fmaxf(__builtin_fmaf(ax, finv.x, nb.x), __builtin_fmaf(ay, finv.y, nb.y)),
-                                   __builtin_fmaf(az, finv.z, nb.z)), tmin);
+                                   __builtin_fmaf(az, finv.z, nb.z)), lo);
       float tf = fminf(fminf(fminf(__builtin_fmaf(bx, finv.x, fb.x), __builtin_fmaf(by, finv.y, fb.y)),
-                             __builtin_fmaf(bz, finv.z, fb.z)), h.t);
+                             __builtin_fmaf(bz, finv.z, fb.z)), hi);
       tf = __builtin_fmaf(fabsf(tf), 0x1p-19f, tf);
       return tn <= tf ? tn : FINF;
     };
@@ -300,7 +329,9 @@ struct Tracer {
 
   // an entry this far away holds nothing nearer than, or as near as, the hit
   PTD bool cull(float etn) const {
-    return etn > (FAST ? __builtin_fmaf(fabsf(h.t), 0x1p-19f, h.t) : h.t);
+    if (!FAST) return etn > h.t;
+    const float t = node_dist(h.t);
+    return etn > __builtin_fmaf(fabsf(t), 0x1p-19f, t);
   }
 
   PTD bool at_node() const { return have && !(ref & LEAF_BIT); }

@@ -1,5 +1,6 @@
 """Rays that meet the conservative node test (the kernels that do not count)
-at its edges, against the exact one (the kernels that count) and the oracle."""
+at its edges, against the exact one (the kernels that count) and the oracle:
+equal distances, origins in the planes of boxes, directions of any length."""
 import sys
 
 import numpy as np
@@ -140,3 +141,52 @@ def test_rays_in_the_planes_of_faces(ctx, mesh):
     differ = ~same(a, b)
     assert (b["inst"] >= 0).mean() > 0.3
     assert not differ.any(), f"{differ.sum()} of {n} rays"
+
+
+# Directions from denormal to almost the largest length: rects, boxes and
+# triangles are met whatever the length (a sphere's or cylinder's square of it
+# overflows or vanishes), as long as the distance itself is a number.  The
+# conservative node test may add a leaf that the exact one's rounding passes
+# by, so it may only be nearer.  Below lengths of 1e-35 the spacing of denormal
+# components (1.4e-45) passes 1e-3 of a rounding (6e-8), so that an instance's
+# ray leaves the world's by what decides a few edges in 30000 rays; there the
+# two tests only have to agree in all but 1e-3.
+@pytest.mark.parametrize("exponent", [-40, -36, -33, -30, -25, -15, 15, 25, 30, 33, 36])
+def test_directions_of_any_length(ctx, exponent):
+    rng = np.random.default_rng(100 + exponent)
+    s, m = faces_at_zero()
+    v, f = icosphere(3, 3.0, (1.0, 2.0, -1.0))
+    s.meshes.append((v, f, None, None, m))
+    for q in range(6):
+        M = np.hstack([np.diag(rng.uniform(0.3, 2.0, 3)), rng.uniform(-6, 6, (3, 1))])
+        s.instance(ptamd.PT_GEOM_MESH, 0, 0, M if q else None)
+    s.rects += [(q % 3, 0, -7.0, 7.0, -7.0, 7.0, float(rng.uniform(-9, 9)), m) for q in range(12)]
+    s.instance(ptamd.PT_GEOM_RECTS, 96, 12)
+    n = 30000
+    k = np.arange(n)
+    org = rng.uniform(-9, 9, (n, 3))
+    unit = rng.normal(size=(n, 3))
+    unit /= np.linalg.norm(unit, axis=1, keepdims=True)
+    rows = k[k % 4 == 1]
+    unit[rows, rng.integers(0, 3, len(rows))] = 0.0
+    d = (unit * 10.0 ** (exponent + rng.uniform(-1, 1, (n, 1)))).astype(np.float32)
+    desc = s.desc()
+    say(f"[gpu] directions of length 1e{exponent}: {n} rays")
+    ctx.set_scene(desc)
+    ctx.build_accel()
+    rays = rays_of(org, d, 0.0)
+    a = ctx.trace_closest(rays)
+    b, _ = ctx.trace_closest(rays, counted=True)
+    differ = ~same(a, b)
+    nearer = (a["t"] < b["t"]) | ((a["t"] == b["t"]) & ((a["inst"] < b["inst"]) |
+                                                       ((a["inst"] == b["inst"]) & (a["prim"] < b["prim"]))))
+    if exponent > -34:
+        assert np.all(~differ | nearer), f"{(differ & ~nearer).sum()} of {n} rays"
+    assert differ.mean() <= 1e-3
+    assert np.array_equal(ctx.trace_occluded(rays), (a["inst"] >= 0).astype(np.uint8))
+    if exponent in (-36, 33):
+        assert (b["inst"] >= 0).mean() > 0.3
+    # with an infinite component the distances along it are zero: a miss
+    d[k, rng.integers(0, 3, n)] = rng.choice([np.inf, -np.inf], n)
+    a = ctx.trace_closest(rays_of(org, d, 1e-3))
+    assert np.all(a["inst"] < 0)
