@@ -51,8 +51,10 @@ PTD void trace_queries(const DevScene& sc, const pt_ray* __restrict__ rays, uint
   if (busy) take();
   uint64_t row = base + stride;  // wave-uniform: the 64 rays being handed out
   uint32_t given = 0;            // of them, handed out
+  uint32_t trips = 0;
   while (true) {
-    if (busy && !tr.step(sc, st, c)) {
+    const bool over = ++trips > TRIPS_MAX;
+    if (busy && (!tr.step(sc, st, c) || over)) {
       done(i);
       busy = false;
     }
@@ -69,6 +71,7 @@ PTD void trace_queries(const DevScene& sc, const pt_ray* __restrict__ rays, uint
       given += (uint32_t)__popcll(idle);
       row += (given >> 6) * stride;
       given &= 63u;
+      trips = 0;
     }
   }
 }
@@ -293,8 +296,10 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(extend_wa
       tr.begin(scene(), mk3(o), mk3(d), tmin, FINF, st, __float_as_uint(o.w), tm);
     };
     if (busy) take(j);
+    uint32_t trips = 0;
     while (true) {
-      if (busy && !tr.step(scene(), st, c)) {
+      const bool over = ++trips > TRIPS_MAX;
+      if (busy && (!tr.step(scene(), st, c) || over)) {
         P.hit[g.pos(j)] = make_float4(tr.h.t, __int_as_float(tr.h.pos), __int_as_float(tr.h.prim), 0.f);
         busy = false;
       }
@@ -311,6 +316,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(extend_wa
           }
         }
         next += (uint32_t)__popcll(idle);
+        trips = 0;
       }
     }
     if (SORT) {

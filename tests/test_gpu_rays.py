@@ -190,3 +190,29 @@ def test_directions_of_any_length(ctx, exponent):
     d[k, rng.integers(0, 3, n)] = rng.choice([np.inf, -np.inf], n)
     a = ctx.trace_closest(rays_of(org, d, 1e-3))
     assert np.all(a["inst"] < 0)
+
+
+# Every traversal loop relies on this to end: children come after their
+# parents, each node has one parent, and every leaf is one the structure owns.
+@pytest.mark.parametrize("cfg,variant", [(ptamd.PT_SCENE_CORNELL, 0), (ptamd.PT_SCENE_RANDOM_SPHERES, 0),
+                                         (ptamd.PT_SCENE_MESHES, 1), (ptamd.PT_SCENE_MESHES, 0),
+                                         (ptamd.PT_SCENE_NEXT_WEEK, 0), (ptamd.PT_SCENE_MOVING_SPHERES, 0)])
+def test_structures_are_trees(ctx, cfg, variant):
+    sc = ptamd.Scene(cfg, 64, 64, variant)
+    say(f"[gpu] structures of scene {cfg} variant {variant}")
+    ctx.set_scene(sc.desc)
+    ctx.build_accel()
+    nodes, _, _, info = ctx.read_accel()
+    parts = [(int(b[0]), int(b[1]), int(b[3])) for b in info]
+    top = max(b + n for b, n, _ in parts)
+    parts.append((top, len(nodes) - top, sc.desc.num_instances))
+    assert sum(n for _, n, _ in parts) == len(nodes)
+    for base, n, prims in parts:
+        child, count = nodes[base:base + n, 24:28].astype(np.int64), nodes[base:base + n, 28:32].astype(np.int64)
+        empty = child == 0xFFFFFFFF
+        inner = ~empty & (count == 0)
+        leaf = ~empty & (count > 0)
+        assert np.all((child > np.arange(n)[:, None]) | ~inner) and np.all((child < n) | ~inner)
+        assert np.array_equal(np.sort(child[inner]), np.arange(1, n))
+        assert np.array_equal(np.sort(np.concatenate([np.arange(f, f + c) for f, c in zip(child[leaf], count[leaf])])),
+                              np.arange(prims))
