@@ -317,6 +317,8 @@ typedef struct pt_render_stats {
   uint32_t cache_plain_batches;  /* batches of this call rendered without
                                     queries because the network had not
                                     passed the judge (new, or failed last)  */
+  uint32_t graph_captures;  /* graphs this call captured (0 when it replayed
+                               an earlier one or launched directly)        */
 } pt_render_stats;
 
 typedef struct pt_accel_stats {

@@ -1377,7 +1377,7 @@ pt_status pt_render(pt_context* c, const pt_render_params* rp, uint32_t frame_be
     if (!c->frame_dev) HIPCHK(c, hipMalloc(&c->frame_dev, 64));
     launch_set_frame(c->frame_dev, frame_begin, c->stream);
   }
-  uint32_t fallbacks = 0, plain_batches = 0;
+  uint32_t fallbacks = 0, plain_batches = 0, captures = 0;
   for (uint32_t f0 = 0; f0 < frame_count; f0 += fpb) {
     uint32_t nf = std::min(fpb, frame_count - f0);
     uint32_t nslots = nf * WH;
@@ -1419,6 +1419,7 @@ pt_status pt_render(pt_context* c, const pt_render_params* rp, uint32_t frame_be
         c->graph = g;
         HIPCHK(c, hipGraphInstantiate(&c->graph_exec, g, nullptr, nullptr, 0));
         c->graph_key = key;
+        captures++;
       }
       HIPCHK(c, hipGraphLaunch(c->graph_exec, c->stream));
       c->last_fpb = nf;
@@ -1545,6 +1546,7 @@ pt_status pt_render(pt_context* c, const pt_render_params* rp, uint32_t frame_be
     out->cache_judge = use_cache ? c->cache_last_judge : -1.0;
     out->cache_fallbacks = use_cache ? c->cache_last_fallbacks : 0u;
     out->cache_plain_batches = use_cache ? c->cache_last_plain_batches : 0u;
+    out->graph_captures = captures;
     if (use_cache && c->cache_last_steps) {
       const uint32_t n = c->cache_last_batch;
       const uint32_t waves = mlp_fwd_bwd_waves(n);
@@ -2019,6 +2021,7 @@ pt_status render_batch_shaped(pt_context* const* ctxs, const pt_render_params* p
       }
     }
   };
+  uint32_t captures = 0;
   if (shape.graph) {
     // replay when everything the captured launches take by value or by
     // address is unchanged: contexts, parameters, frame counts, the scene
@@ -2033,7 +2036,9 @@ pt_status render_batch_shaped(pt_context* const* ctxs, const pt_render_params* p
     add(rcs.data(), n * sizeof(RenderConsts));
     for (uint32_t i = 0; i < n; i++) add(&ctxs[i]->accum, sizeof(double*));
     add(&B->dsc, sizeof(B->dsc));
-    add(&P, sizeof(P));
+    DevPaths pool = P;
+    pool.row = 0;  // each sub-batch's own, set as it is enqueued
+    add(&pool, sizeof(pool));
     const void* ptrs[7] = {B->spill, B->stats, B->d_scenes, B->d_rcs, B->d_item_off, B->d_item_scene, B->d_item_frame};
     add(ptrs, sizeof(ptrs));
     const uint64_t sh[4] = {cap, (uint64_t)sort, (uint64_t)count_trav, (uint64_t)max_depth};
@@ -2051,6 +2056,7 @@ pt_status render_batch_shaped(pt_context* const* ctxs, const pt_render_params* p
       B->batch_graph = g;
       HIPCHK(B, hipGraphInstantiate(&B->batch_graph_exec, g, nullptr, nullptr, 0));
       B->batch_graph_key = key;
+      captures++;
     }
     HIPCHK(B, hipGraphLaunch(B->batch_graph_exec, B->stream));
   } else {
@@ -2096,6 +2102,7 @@ pt_status render_batch_shaped(pt_context* const* ctxs, const pt_render_params* p
     }
     out->extend_launches = (uint32_t)ext_ev.size();
     out->shade_launches = (uint32_t)sh_ev.size();
+    out->graph_captures = captures;
     for (hipEvent_t e : kev) (void)hipEventDestroy(e);
     uint32_t ovf = 0;
     HIPCHK(B, hipMemcpy(&ovf, P.counters + CTR_STACK_OVERFLOW, 4, hipMemcpyDeviceToHost));

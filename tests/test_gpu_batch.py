@@ -148,6 +148,25 @@ def test_batch_graph_replay_is_bit_identical(scenes):
         ctxs[0].sync()
 
 
+def test_batch_graph_is_captured_once(scenes):
+    """Renders of other sizes on the batch's contexts between two equal batches
+    (they lay the shared path pool out in other rows) leave its graph valid;
+    another frame count captures again."""
+    ctxs = [c for _, c in scenes]
+    params = [s.render_params() for s, _ in scenes]
+    params[0] = scenes[0][0].render_params(flags=scenes[0][0].info.flags | ptamd.PT_FLAG_GRAPH)
+    graphs = []
+    for rep in range(4):
+        say(f"[gpu] batch graph, call {rep}")
+        graphs.append(ptamd.render_batch(ctxs, params, [4, 3, 4, 6]).graph_captures)
+        for k in (0, 1):
+            single(*scenes[k], rep + 1)
+    assert graphs == [1, 0, 0, 0]
+    assert ptamd.render_batch(ctxs, params, [5, 3, 4, 8]).graph_captures == 1
+    params[0] = scenes[0][0].render_params()
+    assert ptamd.render_batch(ctxs, params, [5, 3, 4, 8]).graph_captures == 0
+
+
 def test_batch_autotune_picks_a_shape_with_identical_results(scenes):
     frames = [5, 3, 4, 7]
     ctxs = [c for _, c in scenes]
