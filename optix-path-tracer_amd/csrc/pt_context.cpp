@@ -315,20 +315,40 @@ int grid_of(uint64_t n, uint32_t lanes) {
 }
 
 // First bounce of the one launch that runs all the bounces left (SH_TAIL),
-// for a batch of n paths.  Its waves trace lock-step and unsorted, so large
-// sorted batches enter it where a wave holds few paths; unsorted ones and
-// those below 2^23 paths after the camera rays; media, boxes and procedural
-// textures (ext), whose materials diverge most, later.  Measured from bounce
-// 1, 2, 3, 4, 5, 6 on: 1.7 M paths of the sphere scene 1.57, 1.65, 1.71, 1.80,
-// 1.95, 2.09 ms; 2.1 M of the mesh scene 3.29, 3.41, 3.86, 4.16, 4.43, 4.63
-// ms; 1.0 M of the next-week scene (ext) 4.95, 4.25, 3.58, 3.40, 3.60, 3.69
-// ms; 16.8 M of the Cornell box (unsorted) 9.79, 9.93, 10.00, 10.13, 10.16,
-// 10.21 ms; 199 M of the mesh scene 71.7, 63.8, 61.6, 59.8, 59.9, 59.5 ms;
-// 134 M of 16 scenes 58.3, 56.6, 57.1, 57.7, 56.4, 57.8 ms.  With a launch per
-// kernel and bounce throughout these were 4.3, 6.0, 10.5, 10.4, 73 and 70 ms.
-uint32_t tail_depth(uint64_t n, bool sorted, bool ext) {
+// for a batch of n paths.  Its waves trace lock-step and unsorted, so it takes
+// over after the camera rays in batches whose launches are mostly latency, and
+// later where a launch per kernel and bounce has more to give: sorted paths
+// (one program per wave), scenes with meshes (lanes refilled with rays; all
+// the more where one program shades everything, mixed == false), and media,
+// boxes and procedural textures (ext), whose materials diverge most.
+// Measured from bounce 1, 2, 3, 4, 5, 6 on and (last) a launch per kernel and
+// bounce throughout, ms:
+//   spheres, sorted      1.7 M paths   1.57  1.65  1.71  1.80  1.95  2.09  4.3
+//   next week (ext)      1.0 M         4.95  4.25  3.58  3.40  3.60  3.69 10.5
+//   meshes, sorted       2.1 M         2.96  2.67  3.26  3.61  3.93  4.17  5.10
+//                        8.3 M         5.39  4.76  5.04  5.31  5.69  5.97  7.16
+//                         17 M         8.28  7.34  6.92  7.31  7.71  8.04  9.49
+//                        199 M         62.5  56.1  55.2  52.5  52.1  52.6  54.0
+//   meshes, unsorted     8.3 M         5.48  5.57  5.73  5.88  6.07  6.22  7.02
+//                         33 M         13.9  13.6  13.4  13.7  13.8  13.9  14.9
+//                        199 M         62.8  58.9  58.6  57.9  57.9  58.0  59.6
+//   16 scenes, unsorted   18 M         10.8  11.2  11.3  11.2  11.4        14.0
+//                        134 M         59.7  58.8  58.6  58.7  58.7        60.2
+//   meshes, one program  2.1 M         2.30  2.25  2.21  2.32  2.42  2.55  2.78
+//                        8.3 M         6.37  5.89  5.55  5.54  5.61  5.72  6.07
+//                        199 M          112  96.0  87.8  85.5  85.9  86.1  86.4
+//   spheres, unsorted    123 M         41.0  41.1  41.5  41.5  41.7  41.8  43.6
+//   30 k spheres, one     15 M         11.4  11.5  11.5  11.6  11.6  11.5  11.8
+//     program            123 M         80.2  78.6  78.0  77.7  78.0  77.9  78.5
+//   Cornell box, one      17 M         9.60  9.64  9.72  9.76  9.86  9.87  10.2
+//     program            134 M         70.6  69.8  69.1  68.5  68.6  68.6  69.2
+uint32_t tail_depth(uint64_t n, bool sorted, bool ext, bool meshes, bool mixed) {
   if (n < (1u << 18)) return 1u;
-  return ext || (sorted && n >= (1u << 23)) ? 4u : 1u;
+  if (ext) return 4u;
+  const uint64_t many = sorted   ? 1ull << 23
+                        : meshes ? (mixed ? 1ull << 25 : 1ull << 22)
+                                 : (mixed ? ~0ull : 1ull << 26);
+  return n >= many ? 4u : 1u;
 }
 
 // an odd stride near 0.618 n that is coprime to n (a full-period
@@ -1341,7 +1361,8 @@ pt_status pt_render(pt_context* c, const pt_render_params* rp, uint32_t frame_be
     int in = 0, out = 1;
     // with the radiance cache: not before the queries are asked, and not in
     // sorted batches (the sort's order is that of the training records)
-    uint32_t tail = tail_depth(nslots, sort, c->dsc.ext_instances != 0 || (c->mat_types >> PT_MAT_ISOTROPIC) != 0);
+    uint32_t tail = tail_depth(nslots, sort, c->dsc.ext_instances != 0 || (c->mat_types >> PT_MAT_ISOTROPIC) != 0,
+                               (c->dsc.kinds & 8u) != 0, c->shading_kinds > 1);
     if (rc.flags & PT_FLAG_RADIANCE_CACHE) {
       if (rc.cache.query_depth < rp->max_depth) tail = std::max(tail, rc.cache.query_depth + 1);
       if (sort) tail = 0xFFFFFFFFu;
@@ -1842,6 +1863,7 @@ pt_status render_batch_shaped(pt_context* const* ctxs, const pt_render_params* p
   pt_context* B = ctxs[0];
   uint32_t union_types = 0, max_depth = 0;
   bool env = false, ext = false;  // environment MIS; media, cylinders, moving spheres or the normal shader
+  bool meshes = false;
   for (uint32_t i = 0; i < n; i++) {
     pt_context* c = ctxs[i];
     const pt_render_params* rp = params + i;
@@ -1856,6 +1878,7 @@ pt_status render_batch_shaped(pt_context* const* ctxs, const pt_render_params* p
       return fail(B, PT_ERR_INVALID_ARG, "image too large for one batch");
     if (rp->flags & PT_FLAG_RADIANCE_CACHE) return fail(B, PT_ERR_UNSUPPORTED, "no radiance cache in a batch");
     ext = ext || c->dsc.ext_instances != 0 || (c->mat_types >> PT_MAT_ISOTROPIC) != 0;
+    meshes = meshes || (c->dsc.kinds & 8u) != 0;
     union_types |= c->mat_types;
     max_depth = std::max(max_depth, rp->max_depth);
     env = env || ((rp->flags & PT_FLAG_ENV_MIS) && c->dsc.num_lights != c->dsc.num_lights_plain);
@@ -1948,7 +1971,8 @@ pt_status render_batch_shaped(pt_context* const* ctxs, const pt_render_params* p
   }
   const bool want_stats = out != nullptr;
   const bool count_trav = (params[0].flags & PT_FLAG_COUNT_TRAVERSAL) != 0;
-  const bool sort = shape.sort && __builtin_popcount(union_types & ~(1u << PT_MAT_DIFFUSE_LIGHT)) > 1;
+  const bool mixed = __builtin_popcount(union_types & ~(1u << PT_MAT_DIFFUSE_LIGHT)) > 1;  // shading programs
+  const bool sort = shape.sort && mixed;
   const int matset = shade_material_set(union_types);
   DevPaths& P = B->paths;
   launch_fill_u32((uint32_t*)B->stats, (uint64_t)MAX_WAVES * STAT_WORDS * 2, 0u, B->stream);
@@ -1988,7 +2012,7 @@ pt_status render_batch_shaped(pt_context* const* ctxs, const pt_render_params* p
       const BatchStart bs{B->d_rcs, B->d_item_off + k0, B->d_item_scene + k0, B->d_item_frame + k0,
                           (uint32_t)(k1 - k0)};
       int in = 0, o = 1;
-      const uint32_t tail = (count_trav || (params[0].flags & PT_FLAG_DIRECT)) ? 0xFFFFFFFFu : tail_depth(nslots, sort, ext);
+      const uint32_t tail = (count_trav || (params[0].flags & PT_FLAG_DIRECT)) ? 0xFFFFFFFFu : tail_depth(nslots, sort, ext, meshes, mixed);
       for (uint32_t depth = 0; depth < max_depth; depth++) {
         if (depth == tail) {
           hipEvent_t a = kernel_events ? mark() : nullptr;

@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import ptamd
+from helpers import PyScene, icosphere
 
 pytestmark = pytest.mark.gpu
 
@@ -29,6 +30,24 @@ def setup(ctx, cfg, W, H, variant=0):
     ctx.build_accel()
     ctx.set_camera(sc.camera)
     return sc
+
+
+def look_camera(origin, W, H, vfov=40.0):
+    """Pinhole camera at `origin` looking at 0, up +y."""
+    o = np.array(origin, np.float64)
+    w = o / np.linalg.norm(o)
+    u = np.cross([0, 1, 0], w)
+    u /= np.linalg.norm(u)
+    v = np.cross(w, u)
+    hh = np.tan(np.radians(vfov) / 2)
+    hw = hh * W / H
+    c = ptamd.Camera()
+    c.origin[:] = o
+    c.lower_left[:] = o - hw * u - hh * v - w
+    c.horizontal[:] = 2 * hw * u
+    c.vertical[:] = 2 * hh * v
+    c.u[:], c.v[:], c.w[:] = u, v, w
+    return c
 
 
 def image(ctx, params, f0, n):
@@ -130,3 +149,51 @@ def test_last_bounces_in_one_launch_are_bit_identical(ctx, cfg, W, H, frames, de
                         np.array([st.extension_rays, st.shadow_rays, st.exhausted_paths, st.nan_paths])))
         for a, b in zip(*got):
             assert np.array_equal(a, b, equal_nan=True)
+
+
+def one_program_meshes():
+    """Meshes and a ground rect of one Lambertian material."""
+    s = PyScene()
+    m = s.lambert((0.6, 0.6, 0.6))
+    v, f = icosphere(4)
+    s.meshes.append((v, f, None, None, m))
+    rng = np.random.default_rng(0)
+    for _ in range(12):
+        s.instance(ptamd.PT_GEOM_MESH, 0, 0, np.hstack([np.eye(3) * rng.uniform(0.5, 1.5), rng.uniform(-5, 5, (3, 1))]))
+    s.rects.append((1, 0, -50.0, 50.0, -50.0, 50.0, -6.0, m))
+    s.instance(ptamd.PT_GEOM_RECTS, 0, 1)
+    return s
+
+
+# The bounce from which one launch runs the rest (extend_launches), on both
+# sides of each of the rule's sizes, and the same image, ray counts and path
+# ends as a launch per kernel and bounce gives.
+@pytest.mark.parametrize("cfg,sort,W,H,frames,first", [
+    (ptamd.PT_SCENE_MESHES, False, 1000, 2097, 16, 1), (ptamd.PT_SCENE_MESHES, False, 1024, 2049, 16, 4),
+    (ptamd.PT_SCENE_MESHES, True, 1000, 1047, 8, 1), (ptamd.PT_SCENE_MESHES, True, 1024, 1025, 8, 4),
+    ("one program", False, 1000, 1047, 4, 1), ("one program", False, 1024, 1025, 4, 4),
+    (ptamd.PT_SCENE_CORNELL, True, 1000, 1047, 64, 1), (ptamd.PT_SCENE_CORNELL, True, 1024, 1025, 64, 4),
+    (ptamd.PT_SCENE_RANDOM_SPHERES, False, 1024, 1025, 64, 1), (ptamd.PT_SCENE_RANDOM_SPHERES, True, 1024, 1025, 8, 4),
+    (ptamd.PT_SCENE_NEXT_WEEK, True, 512, 511, 1, 1), (ptamd.PT_SCENE_NEXT_WEEK, False, 513, 512, 1, 4)])
+def test_where_the_last_bounces_launch_begins(ctx, cfg, sort, W, H, frames, first):
+    if cfg == "one program":
+        s = one_program_meshes()
+        ctx.set_scene(s.desc())
+        ctx.build_accel()
+        ctx.set_camera(look_camera((0.8, 1.5, 14.0), W, H))
+        make = lambda flags: ptamd.RenderParams(W, H, 8, 1, 3, 0, flags, 0)  # noqa: E731
+        base = 0
+    else:
+        sc = setup(ctx, cfg, W, H, 3 if cfg == ptamd.PT_SCENE_MESHES else 0)
+        make = lambda flags: sc.render_params(flags=flags)  # noqa: E731
+        base = sc.info.flags & ~ptamd.PT_FLAG_MATERIAL_SORT
+    if sort:
+        base |= ptamd.PT_FLAG_MATERIAL_SORT
+    say(f"[gpu] last bounces of {W * H * frames} paths, scene {cfg}, sort {sort}")
+    a, sa = image(ctx, make(base), 0, frames)
+    b, sb = image(ctx, make(base | ptamd.PT_FLAG_DIRECT), 0, frames)
+    assert sa.extend_launches == first and sa.shade_launches == first + 1
+    assert sb.extend_launches == sb.shade_launches == make(base).max_depth
+    assert np.array_equal(a, b)
+    for k in ("extension_rays", "shadow_rays", "exhausted_paths", "nan_paths"):
+        assert getattr(sa, k) == getattr(sb, k), k
