@@ -6,7 +6,6 @@ namespace pt {
 void launch_shade(const DevScene& sc, const DevPaths& P, int in, bool sorted, int out, uint32_t depth,
                   const RenderConsts& rc, int matset, bool count, uint2* spill, uint64_t* stats, int grid,
                   hipStream_t st, const DevScene* scenes, const RenderConsts* rcs, bool batch_env, bool batch_ext) {
-  if (!scenes && sc.wide) count = true;
   const int src = sorted ? 2 : in;
   const float4* hits = sorted ? P.hit_sorted : P.hit;
   const bool env = (rc.flags & PT_FLAG_ENV_MIS) && sc.num_lights != sc.num_lights_plain;
@@ -31,6 +30,10 @@ void launch_shade(const DevScene& sc, const DevPaths& P, int in, bool sorted, in
       if (count) PT_SHADE(MS_ALL, SH_MULTI | SH_COUNT);
       else PT_SHADE(MS_ALL, SH_MULTI);
     }
+  } else if (sc.wide && (!count || cache)) {  // few scenes: every material and both kinds of lights
+    if (matset == MS_FULL || sc.ext_instances != 0) PT_SHADE(MS_FULL, SH_WIDE | SH_EXT | SH_ENV);
+    else if (cache) PT_SHADE(MS_ALL, SH_WIDE | SH_CACHE | SH_ENV);
+    else PT_SHADE(MS_ALL, SH_WIDE | SH_ENV);
   } else if (matset == MS_FULL || sc.ext_instances != 0) {
     // media or the normal shader (single scenes, no radiance cache)
     if (env) {
@@ -40,9 +43,6 @@ void launch_shade(const DevScene& sc, const DevPaths& P, int in, bool sorted, in
       if (count) PT_SHADE(MS_FULL, SH_EXT | SH_COUNT);
       else PT_SHADE(MS_FULL, SH_EXT);
     }
-  } else if (cache && sc.wide) {  // every material
-    if (env) PT_SHADE(MS_ALL, SH_CACHE | SH_ENV | SH_COUNT);
-    else PT_SHADE(MS_ALL, SH_CACHE | SH_COUNT);
   } else if (cache) {  // not asked to count
     if (env) PT_SHADE(MS_ALL, SH_CACHE | SH_ENV);
     else PT_SHADE(MS_ALL, SH_CACHE);

@@ -1367,7 +1367,7 @@ pt_status pt_render(pt_context* c, const pt_render_params* rp, uint32_t frame_be
       if (rc.cache.query_depth < rp->max_depth) tail = std::max(tail, rc.cache.query_depth + 1);
       if (sort) tail = 0xFFFFFFFFu;
     }
-    if (count_trav || c->dsc.wide || (rp->flags & PT_FLAG_DIRECT)) tail = 0xFFFFFFFFu;
+    if (count_trav || (rp->flags & PT_FLAG_DIRECT)) tail = 0xFFFFFFFFu;
     for (uint32_t depth = 0; depth < rp->max_depth; depth++) {
       if (depth == tail) {
         hipEvent_t a = events ? mark() : nullptr;
@@ -1550,14 +1550,12 @@ pt_status pt_render(pt_context* c, const pt_render_params* rp, uint32_t frame_be
     out->paths = (uint64_t)frame_count * WH;
     out->extension_rays = st[STAT_EXT];
     out->shadow_rays = st[STAT_SHADOW];
-    if (count_trav) {  // (wide scenes always count)
-      out->node_fetches = st[STAT_NODES];
-      out->prim_fetches = st[STAT_PRIMS];
-      out->instance_fetches = st[STAT_INSTS];
-      out->shadow_node_fetches = st[STAT_SH_NODES];
-      out->shadow_prim_fetches = st[STAT_SH_PRIMS];
-      out->shadow_instance_fetches = st[STAT_SH_INSTS];
-    }
+    out->node_fetches = st[STAT_NODES];
+    out->prim_fetches = st[STAT_PRIMS];
+    out->instance_fetches = st[STAT_INSTS];
+    out->shadow_node_fetches = st[STAT_SH_NODES];
+    out->shadow_prim_fetches = st[STAT_SH_PRIMS];
+    out->shadow_instance_fetches = st[STAT_SH_INSTS];
     out->exhausted_paths = st[STAT_EXHAUSTED];
     out->nan_paths = st[STAT_NAN];
     out->cache_queries = c->cache_last_query;

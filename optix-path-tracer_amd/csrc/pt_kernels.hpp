@@ -31,9 +31,9 @@ struct RenderConsts {
   uint32_t store_time;        // keep each path's ray time (the scene has moving spheres)
 };
 
-// Render path (pt_render.hip, pt_bounce.hip, pt_tail.hip).  Scenes whose
-// nodes take 4 GB or more (DevScene::wide) run the counting kernels, whose
-// node addresses are 64-bit.
+// Render path (pt_render.hip, pt_bounce.hip, pt_tail.hip).  A scene whose
+// nodes take 4 GB or more (DevScene::wide) runs kernels of its own with 64-bit
+// node addresses, as those of a batch and those that count have throughout.
 void launch_trace_closest(const DevScene& sc, const pt_ray* rays, uint64_t n, pt_hit* hits, uint32_t* counts,
                           uint2* spill, uint32_t* overflow, int grid, hipStream_t st);
 void launch_trace_occluded(const DevScene& sc, const pt_ray* rays, uint64_t n, uint8_t* occ, uint2* spill,

@@ -76,13 +76,13 @@ PTD void trace_queries(const DevScene& sc, const pt_ray* __restrict__ rays, uint
   }
 }
 
-template <bool COUNT, bool EXT, bool REFILL>
+template <bool COUNT, bool EXT, bool REFILL, bool WIDE>
 __global__ __launch_bounds__(BLOCK) void k_trace_closest(DevScene sc, const pt_ray* __restrict__ rays, uint64_t n,
                                                          pt_hit* __restrict__ hits, uint32_t* __restrict__ counts,
                                                          uint2* spill, uint32_t* overflow) {
   __shared__ uint2 s_stk[STK_LDS * BLOCK];
   Stack st = make_stack(s_stk, spill, overflow);
-  Tracer<COUNT, EXT, KIND_ALL, false, false, true> tr;
+  Tracer<COUNT, EXT, KIND_ALL, false, WIDE, true> tr;
   TraceCounts c;
   trace_queries<EXT, REFILL>(sc, rays, n, st, tr, c, [&](uint64_t i) {
     const HitOut& h = tr.h;
@@ -92,7 +92,7 @@ __global__ __launch_bounds__(BLOCK) void k_trace_closest(DevScene sc, const pt_r
     out.prim = h.prim;
     out.reserved = 0;
     hits[i] = out;
-    if (COUNT && counts) {
+    if (COUNT) {
       counts[3 * i + 0] = c.nodes;
       counts[3 * i + 1] = c.prims;
       counts[3 * i + 2] = c.insts;
@@ -100,13 +100,13 @@ __global__ __launch_bounds__(BLOCK) void k_trace_closest(DevScene sc, const pt_r
   });
 }
 
-template <bool COUNT, bool EXT, bool REFILL>
+template <bool COUNT, bool EXT, bool REFILL, bool WIDE>
 __global__ __launch_bounds__(BLOCK) void k_trace_occluded(DevScene sc, const pt_ray* __restrict__ rays, uint64_t n,
                                                           uint8_t* __restrict__ occ, uint2* spill,
                                                           uint32_t* overflow) {
   __shared__ uint2 s_stk[STK_LDS * BLOCK];
   Stack st = make_stack(s_stk, spill, overflow);
-  Tracer<COUNT, EXT, KIND_ALL, false, false, true> tr;
+  Tracer<COUNT, EXT, KIND_ALL, false, WIDE, true> tr;
   TraceCounts c;
   trace_queries<EXT, REFILL>(sc, rays, n, st, tr, c, [&](uint64_t i) {
     const HitOut& h = tr.h;
@@ -247,12 +247,12 @@ PTD uint32_t material_key(const DevScene& sc, float4 h) {
 // instead of 10.2 ms and the mesh still 67.3 instead of 65.1 ms; a batch of
 // 16 scenes took 66.6 ms with both and its bounce rays at 5, 65.4 ms with the
 // latter alone, 63.6 ms with neither.
-template <int KINDS, bool START, bool MULTI>
-constexpr int extend_waves() { return START || MULTI ? 4 : PT_EXTEND_WAVES; }
+template <int KINDS, bool START, bool WIDE>
+constexpr int extend_waves() { return START || WIDE ? 4 : PT_EXTEND_WAVES; }
 template <int KINDS>
 constexpr int extend_stk() { return (KINDS & 8) ? STK_LDS_EXTEND : 12; }
-template <bool COUNT, bool SORT, bool MULTI, bool EXT, int KINDS = KIND_ALL, bool START = false>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(extend_waves<KINDS, START, MULTI>(), 8))) void k_extend(
+template <bool COUNT, bool SORT, bool MULTI, bool EXT, int KINDS = KIND_ALL, bool START = false, bool WIDE = MULTI>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(extend_waves<KINDS, START, WIDE>(), 8))) void k_extend(
     DevScene sc0, DevPaths P, int in, float tmin, uint2* spill, uint64_t* stats, const DevScene* __restrict__ scenes,
     RenderConsts rc, uint32_t nstart, BatchStart bs) {
   constexpr int NS = extend_stk<KINDS>();
@@ -283,7 +283,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(extend_wa
     // lanes' steps stay alike.)  In a batch of scenes each lane keeps its
     // scene (16 scenes 59.1 -> 58.7 ms per pass, and 57.8 ms with the node
     // array's address kept per ray and the table's pointers known as global).
-    Tracer<COUNT, EXT, KINDS, false, MULTI> tr;
+    Tracer<COUNT, EXT, KINDS, false, WIDE> tr;
     uint32_t j = __lane_id(), sid = 0;
     auto scene = [&]() -> const DevScene& { return MULTI ? scenes[sid] : sc0; };
     bool busy = j < n;
@@ -368,7 +368,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(extend_wa
       }
       const DevScene& sc = MULTI ? scenes[__float_as_uint(o.w) >> 24] : sc0;
       if (EXT && sc.mov_instances && !starts) tm = P.ptime[__float_as_uint(d.w) & SLOT_MASK];
-      HitOut h = trace_closest<COUNT, EXT, KINDS, false, MULTI>(sc, mk3(o), mk3(d), tmin, FINF, st, c, __float_as_uint(o.w), tm);
+      HitOut h = trace_closest<COUNT, EXT, KINDS, false, WIDE>(sc, mk3(o), mk3(d), tmin, FINF, st, c, __float_as_uint(o.w), tm);
       float4 hv = make_float4(h.t, __int_as_float(h.pos), __int_as_float(h.prim), 0.f);
       P.hit[i] = hv;
       if (SORT) {
@@ -734,34 +734,37 @@ __global__ void k_fill_f64(double* p, uint64_t n, double v) {
 // --------------------------------------------------------- host launchers
 void launch_trace_closest(const DevScene& sc, const pt_ray* rays, uint64_t n, pt_hit* hits, uint32_t* counts,
                           uint2* spill, uint32_t* overflow, int grid, hipStream_t st) {
-#define PT_TRACE(C, V, R)                                                                                       \
-  hipLaunchKernelGGL((k_trace_closest<C, V, R>), dim3(grid), dim3(BLOCK), 0, st, sc, rays, n, hits, counts, spill, \
+#define PT_TRACE(C, V, R, W)                                                                                       \
+  hipLaunchKernelGGL((k_trace_closest<C, V, R, W>), dim3(grid), dim3(BLOCK), 0, st, sc, rays, n, hits, counts, spill, \
                      overflow)
   const bool vol = sc.ext_instances != 0, refill = (sc.kinds & 8u) != 0;
-  if (counts || sc.wide) {
-    if (vol) PT_TRACE(true, true, false);
-    else PT_TRACE(true, false, false);
+  if (counts) {
+    if (vol) PT_TRACE(true, true, false, false);
+    else PT_TRACE(true, false, false, false);
+  } else if (sc.wide) {
+    if (vol) PT_TRACE(false, true, false, true);
+    else PT_TRACE(false, false, true, true);
   } else if (vol) {
-    PT_TRACE(false, true, false);
+    PT_TRACE(false, true, false, false);
   } else if (refill) {
-    PT_TRACE(false, false, true);
+    PT_TRACE(false, false, true, false);
   } else {
-    PT_TRACE(false, false, false);
+    PT_TRACE(false, false, false, false);
   }
 #undef PT_TRACE
 }
 void launch_trace_occluded(const DevScene& sc, const pt_ray* rays, uint64_t n, uint8_t* occ, uint2* spill,
                            uint32_t* overflow, int grid, hipStream_t st) {
-#define PT_OCC(C, V, R) \
-  hipLaunchKernelGGL((k_trace_occluded<C, V, R>), dim3(grid), dim3(BLOCK), 0, st, sc, rays, n, occ, spill, overflow)
+#define PT_OCC(V, R, W) \
+  hipLaunchKernelGGL((k_trace_occluded<false, V, R, W>), dim3(grid), dim3(BLOCK), 0, st, sc, rays, n, occ, spill, overflow)
   const bool vol = sc.ext_instances != 0, refill = (sc.kinds & 8u) != 0;
   if (sc.wide) {
-    if (vol) PT_OCC(true, true, false);
-    else PT_OCC(true, false, false);
+    if (vol) PT_OCC(true, false, true);
+    else PT_OCC(false, true, true);
   } else if (vol) {
-    PT_OCC(false, true, false);
+    PT_OCC(true, false, false);
   } else if (refill) {
-    PT_OCC(false, false, true);
+    PT_OCC(false, true, false);
   } else {
     PT_OCC(false, false, false);
   }
@@ -785,7 +788,6 @@ static int extend_kinds(uint32_t k) {
 void launch_extend(const DevScene& sc, const DevPaths& P, int in, float tmin, uint2* spill, uint64_t* stats,
                    bool count_traversal, bool sort, int grid, hipStream_t st, const DevScene* scenes,
                    const RenderConsts* start, uint32_t nstart, bool multi_ext, const BatchStart* bstart) {
-  if (!scenes && sc.wide) count_traversal = true;
   const RenderConsts rc = start ? *start : RenderConsts{};
   const bool starts = start != nullptr && scenes == nullptr && nstart != 0;
   const bool bstarts = bstart != nullptr && scenes != nullptr && nstart != 0 && bstart->nitems != 0;
@@ -820,7 +822,23 @@ void launch_extend(const DevScene& sc, const DevPaths& P, int in, float tmin, ui
       }                                                                                                  \
     }                                                                                                    \
   } while (0)
-  if (bstarts && multi_ext) {
+  // One scene of 4 GB of nodes or more (it has meshes: nothing else comes
+  // near).  218 M triangles, 1080p at 8 spp: 32.1 ms with the counting kernels,
+  // 28.3 ms with these; 4 M rays 4.84 -> 4.45 ms.
+#define PT_EXTEND_WIDE(S, ST)                                                                                       \
+  do {                                                                                                              \
+    if (sc.ext_instances != 0)                                                                                      \
+      hipLaunchKernelGGL((k_extend<false, S, false, true, KIND_ALL, ST, true>), dim3(grid), dim3(BLOCK), 0, st, sc, \
+                         P, in, tmin, spill, stats, scenes, rc, nstart, bs);                                        \
+    else                                                                                                            \
+      hipLaunchKernelGGL((k_extend<false, S, false, false, KIND_ALL, ST, true>), dim3(grid), dim3(BLOCK), 0, st,    \
+                         sc, P, in, tmin, spill, stats, scenes, rc, nstart, bs);                                    \
+  } while (0)
+  if (!scenes && sc.wide && !count_traversal) {
+    if (starts) PT_EXTEND_WIDE(false, true);
+    else if (sort) PT_EXTEND_WIDE(true, false);
+    else PT_EXTEND_WIDE(false, false);
+  } else if (bstarts && multi_ext) {
     PT_EXTEND2(true, true, KIND_ALL, true);
   } else if (bstarts) {
     PT_EXTEND2(true, false, KIND_ALL, true);
@@ -833,6 +851,7 @@ void launch_extend(const DevScene& sc, const DevPaths& P, int in, float tmin, ui
   } else {
     PT_EXTEND_KINDS(false, PT_EXTEND4);
   }
+#undef PT_EXTEND_WIDE
 #undef PT_EXTEND_KINDS
 #undef PT_EXTEND2
 #undef PT_EXTEND4

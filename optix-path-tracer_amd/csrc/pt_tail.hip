@@ -15,6 +15,10 @@ void launch_tail(const DevScene& sc, const DevPaths& P, int in, int out, uint32_
   } else if (scenes) {
     if (batch_env) PT_TAIL(MS_ALL, SH_MULTI | SH_ENV, KIND_ALL);
     else PT_TAIL(MS_ALL, SH_MULTI, KIND_ALL);
+  } else if (sc.wide) {
+    if (matset == MS_FULL || sc.ext_instances != 0) PT_TAIL(MS_FULL, SH_WIDE | SH_EXT | SH_ENV, KIND_ALL);
+    else if (rc.flags & PT_FLAG_RADIANCE_CACHE) PT_TAIL(MS_ALL, SH_WIDE | SH_CACHE | SH_ENV, KIND_ALL);
+    else PT_TAIL(MS_ALL, SH_WIDE | SH_ENV, KIND_ALL);
   } else if (matset == MS_FULL || sc.ext_instances != 0) {
     if (env) PT_TAIL(MS_FULL, SH_EXT | SH_ENV, KIND_ALL);
     else PT_TAIL(MS_FULL, SH_EXT, KIND_ALL);

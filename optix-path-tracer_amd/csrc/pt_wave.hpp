@@ -251,7 +251,8 @@ PTD bool scatter_and_roulette(const Surface& f, v3 Wo, v3 N, uint32_t& seed, uin
 // 1.9 ms, next-week scene 10.5 -> 4.1 ms, one 1080p frame of the mesh scene
 // 6.0 -> 4.6 ms (257 us, 1.4, 3.4 and 3.4 ms with the traversal and the
 // spread of small batches of today).
-constexpr int SH_COUNT = 1, SH_CACHE = 2, SH_ENV = 4, SH_MULTI = 8, SH_EXT = 16, SH_TAIL = 32;
+// SH_WIDE: 64-bit node addresses (one scene of 4 GB of nodes or more).
+constexpr int SH_COUNT = 1, SH_CACHE = 2, SH_ENV = 4, SH_MULTI = 8, SH_EXT = 16, SH_TAIL = 32, SH_WIDE = 64;
 template <int MS, int FEAT, int KINDS = KIND_ALL>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_shade(
     DevScene sc0, DevPaths P, int in, int src, const float4* __restrict__ hits, int out, uint32_t depth0,
@@ -259,6 +260,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
     const RenderConsts* __restrict__ rcs) {
   constexpr bool MULTI = (FEAT & SH_MULTI) != 0;
   constexpr bool EXT = (FEAT & SH_EXT) != 0;
+  constexpr bool WIDE = (FEAT & (SH_MULTI | SH_WIDE)) != 0;
   __shared__ uint2 s_stk[STK_LDS_SHADE * BLOCK];
   // each lane's T, L, normal and view direction wait here while its shadow
   // ray is traced: fewer registers live across the traversal (fewer scratch
@@ -298,7 +300,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
         if (TAIL) {
           const DevScene& tsc = MULTI ? scenes[__float_as_uint(o4.w) >> 24] : sc0;
           const float ttm = (EXT && tsc.mov_instances) ? P.ptime[__float_as_uint(d4.w) & SLOT_MASK] : 0.f;
-          const HitOut th = trace_closest<false, EXT, KINDS, false, MULTI>(tsc, mk3(o4), mk3(d4), 1e-3f, FINF, st, tc,
+          const HitOut th = trace_closest<false, EXT, KINDS, false, WIDE>(tsc, mk3(o4), mk3(d4), 1e-3f, FINF, st, tc,
                                                              __float_as_uint(o4.w), ttm);
           hit = make_float4(th.t, __int_as_float(th.pos), __int_as_float(th.prim), 0.f);
         } else {
@@ -408,7 +410,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
                   keep(9, r.Wo);
                   // an environment sample is lit iff its shadow ray hits
                   // nothing (any hit occludes): the first hit found decides it
-                  HitOut sh = trace_closest<COUNT, EXT, KINDS, true, MULTI>(sc, r.P, Wi, 1e-3f, FINF, st, tc, seed, tm, env);
+                  HitOut sh = trace_closest<COUNT, EXT, KINDS, true, WIDE>(sc, r.P, Wi, 1e-3f, FINF, st, tc, seed, tm, env);
                   T = kept(0);
                   L = kept(3);
                   r.N = kept(6);
@@ -503,7 +505,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
       // fence makes what other lanes stored visible to the next loads
       __threadfence_block();
       n = survivors;
-      const PathState X = depth == depth0 ? P.st[in] : S;
+      const PathState X = S;
       S = D;
       D = X;
       depth++;
