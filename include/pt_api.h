@@ -497,14 +497,17 @@ pt_status pt_autotune(struct pt_context* ctx, const pt_render_params* params, ui
 
 /* No counterpart in the reference.  The same for a batch of scenes: renders
  * the batch (pt_render_batch semantics, with the given frame counts, which
- * may be fewer than the production render's) under 8, 16, 32, 64, 128 and
- * 256 Mi paths per sub-batch (at most the automatic batch size) x material
- * sort on/off (when the batch has more than
- * one shading program) x graph replay on/off, twice each, and keeps the
- * fastest second run in ctxs[0] for pt_render_batch calls whose params[0]
- * has PT_FLAG_TUNED and whose contexts and parameters (other than the
- * shape's own flags and frames_per_batch) are the same.  Every context's
- * accumulation is left holding the tuning render. */
+ * may be fewer than the production render's) in the default even
+ * sub-batches and under 8, 16, 32, 64, 128 and 256 Mi paths per sub-batch (at
+ * most the automatic batch size, and where they cut the given counts
+ * otherwise) x material sort on/off (when the batch has more than one shading
+ * program) x graph replay on/off, twice each.  The fastest second run is kept
+ * in ctxs[0] (a fixed size when it is 5 % faster than the even sub-batches,
+ * which adapt to the production render's counts; paths_per_batch is 2^27 for
+ * those) for pt_render_batch calls whose params[0] has PT_FLAG_TUNED and whose
+ * contexts and parameters (other than the shape's own flags and
+ * frames_per_batch) are the same.  Every context's accumulation is left
+ * holding the tuning render. */
 pt_status pt_autotune_batch(struct pt_context* const* ctxs, const pt_render_params* params,
                             const uint32_t* frame_counts, uint32_t n, pt_tune_result* out_or_null);
 

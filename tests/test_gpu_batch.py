@@ -187,6 +187,30 @@ def test_batch_autotune_picks_a_shape_with_identical_results(scenes):
         assert np.array_equal(c.read_accum(s.info.width, s.info.height)[0], d)
 
 
+def test_tuned_batch_keeps_the_even_parts():
+    """Tuned on frame counts that every candidate size takes at once, the
+    production batch of 208 M paths still runs in the untuned batch's two
+    parts."""
+    made = [make(ptamd.PT_SCENE_CORNELL, 1024, 1024), make(ptamd.PT_SCENE_RANDOM_SPHERES, 400, 267)]
+    try:
+        ctxs = [c for _, c in made]
+        frames = [198, 3]
+        params = [s.render_params() for s, _ in made]
+        for p in params:
+            p.max_depth = 4
+        say("[gpu] tune a batch on 2 + 1 frames")
+        assert ptamd.autotune_batch(ctxs, params, [2, 1]).candidates == 4
+        launches = []
+        for extra in (0, ptamd.PT_FLAG_TUNED):
+            p = [ptamd.RenderParams.from_buffer_copy(q) for q in params]
+            p[0].flags |= ptamd.PT_FLAG_DIRECT | extra
+            launches.append(ptamd.render_batch(ctxs, p, frames).shade_launches)
+        assert launches == [2 * 4, 2 * 4]
+    finally:
+        for _, ctx in made:
+            ctx.close()
+
+
 # the 64-scene workload's largest mesh scenes (1.31 M and 1.18 M triangles),
 # its largest sphere scene (4478 spheres) and five more, at full resolution
 C3_SUBSET = [49, 63, 44, 33, 20, 1, 11, 7]
