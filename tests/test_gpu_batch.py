@@ -294,6 +294,37 @@ def test_large_batch_in_even_parts():
             ctx.close()
 
 
+# the last bounces' launch begins after the camera rays (few paths), at bounce
+# 4 (sorted from 2^23 paths on, media from 2^18 on); depths on both sides
+@pytest.mark.parametrize("media,frames,depths,first", [
+    (False, (5, 3, 4), (1, 2, 12), 1), (False, (130, 60, 3), (4, 5, 12), 4), (True, (2, 3, 1), (1, 2, 9), 1),
+    (True, (60, 60, 10), (4, 5, 9), 4)])
+def test_batch_last_bounces_in_one_launch(media, frames, depths, first):
+    """Against a launch per kernel and bounce: the same images and counts."""
+    kinds = ((ptamd.PT_SCENE_NEXT_WEEK, 48, 48, 0), (ptamd.PT_SCENE_MOVING_SPHERES, 61, 47, 0)) if media else \
+        ((ptamd.PT_SCENE_RANDOM_SPHERES, 256, 192, 0), (ptamd.PT_SCENE_CORNELL, 200, 200, 0))
+    made = [make(*k) for k in kinds + ((ptamd.PT_SCENE_MESHES, 160, 90, 5),)]
+    try:
+        ctxs = [c for _, c in made]
+        for depth in depths:
+            say(f"[gpu] batch, media {media}, frames {frames}, depth {depth}")
+            got = []
+            for extra in (0, ptamd.PT_FLAG_DIRECT):
+                params = [s.render_params() for s, _ in made]
+                for k, p in enumerate(params):
+                    p.max_depth = max(1, depth - k)  # scenes of unequal depths
+                params[0].flags |= extra | ptamd.PT_FLAG_MATERIAL_SORT
+                st = ptamd.render_batch(ctxs, params, frames)
+                assert st.extend_launches == (depth if extra else min(depth, first))
+                got.append([c.read_accum(s.info.width, s.info.height)[0] for s, c in made] +
+                           [np.array([st.extension_rays, st.shadow_rays, st.exhausted_paths, st.nan_paths])])
+            for a, b in zip(*got):
+                assert np.array_equal(a, b)
+    finally:
+        for _, ctx in made:
+            ctx.close()
+
+
 def test_batch_rejects_bad_input(scenes):
     sc, ctx = scenes[0]
     p = sc.render_params()

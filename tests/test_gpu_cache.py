@@ -221,6 +221,49 @@ def test_queries_end_paths_and_training_converges(ctx):
     assert escaped < 0.3 * third.size, (escaped, third.size)
 
 
+# held (a new network: the last bounces' launch begins after the camera rays)
+# and answered (it begins after the query depth), unsorted; sorted batches keep
+# a launch per kernel and bounce
+@pytest.mark.parametrize("answered", [False, True])
+@pytest.mark.parametrize("query_depth", [0, 2, 15])
+@pytest.mark.parametrize("meshes", [False, True])
+def test_cached_frames_in_any_launch_shape(ctx, meshes, query_depth, answered):
+    """One launch for the last bounces against a launch per kernel and bounce:
+    the same records in the same order, hence the same network, image and
+    counts."""
+    say(f"[gpu] cached frames, meshes {meshes}, query depth {query_depth}, answered {answered}")
+    if meshes:
+        W, H = 160, 90
+        sc = ptamd.Scene(ptamd.PT_SCENE_MESHES, W, H, 4)
+        ctx.set_scene(sc.desc)
+        ctx.build_accel()
+        ctx.set_camera(sc.camera)
+    else:
+        W, H = 97, 61
+        sc = cornell(ctx, W, H)
+    flags = (sc.info.flags & ~ptamd.PT_FLAG_MATERIAL_SORT) | ptamd.PT_FLAG_KEEP_PATHS | ptamd.PT_FLAG_RADIANCE_CACHE
+    ctx.cache_configure(query_depth=query_depth, train_fraction=0.2, batch=2048, steps=3)
+    ctx.cache_judge_configure(max_ratio=1e30 if answered else 0.0)
+    got = []
+    try:
+        for extra in (0, ptamd.PT_FLAG_DIRECT):
+            ctx.cache_init(9)
+            st = ctx.render(sc.render_params(flags=flags | extra, frames_per_batch=1), 0, 3)
+            assert st.cache_plain_batches == (1 if answered else 3)
+            got.append([ctx.read_accum(W, H)[0], *ctx.read_paths(W, H), *ctx.cache_records(0)[:3],
+                        *ctx.cache_records(1)[:3], ctx.cache_params(),
+                        np.array([st.extension_rays, st.shadow_rays, st.exhausted_paths, st.cache_queries,
+                                  st.cache_train_vertices, st.cache_loss])])
+            launches = st.extend_launches
+        assert launches == 3 * sc.info.max_depth
+    finally:
+        ctx.cache_judge_configure()
+        ctx.cache_configure()
+    assert len(got[0][4]) > 500
+    for a, b in zip(*got):
+        assert np.array_equal(a, b, equal_nan=True)
+
+
 def test_judge_fallback_renders_the_plain_image(ctx):
     """A new network is held: until the judge passes it, batches render
     plain (no queries; training paths still train).  A judge that passes

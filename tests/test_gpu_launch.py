@@ -197,3 +197,17 @@ def test_where_the_last_bounces_launch_begins(ctx, cfg, sort, W, H, frames, firs
     assert np.array_equal(a, b)
     for k in ("extension_rays", "shadow_rays", "exhausted_paths", "nan_paths"):
         assert getattr(sa, k) == getattr(sb, k), k
+
+
+# The kernels that count use the exact node test: the same hits, hence images.
+@pytest.mark.parametrize("cfg,variant,W,H,frames", [
+    (ptamd.PT_SCENE_RANDOM_SPHERES, 0, 400, 267, 16), (ptamd.PT_SCENE_CORNELL, 0, 256, 256, 16),
+    (ptamd.PT_SCENE_MESHES, 5, 480, 270, 8), (ptamd.PT_SCENE_NEXT_WEEK, 0, 301, 203, 8),
+    (ptamd.PT_SCENE_MOVING_SPHERES, 0, 301, 203, 8)])
+def test_counting_kernels_render_the_same_image(ctx, cfg, variant, W, H, frames):
+    sc = setup(ctx, cfg, W, H, variant)
+    say(f"[gpu] default and counting image, scene {cfg}")
+    a, sa = image(ctx, sc.render_params(), 0, frames)
+    b, sb = image(ctx, sc.render_params(flags=sc.info.flags | ptamd.PT_FLAG_COUNT_TRAVERSAL), 0, frames)
+    assert np.array_equal(a, b)
+    assert (sa.extension_rays, sa.shadow_rays) == (sb.extension_rays, sb.shadow_rays)
