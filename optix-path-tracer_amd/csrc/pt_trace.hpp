@@ -4,8 +4,8 @@
 // One ray per lane.  The traversal stack keeps its top entries in LDS (one
 // column per lane, bank-conflict free; how many is the kernel's choice) and
 // spills deeper entries to a per-thread slice of HBM.  Children are visited
-// nearest first by entry distance; popped entries farther than the current hit
-// are skipped (with node_fast's margin where its distances are compared).
+// nearest first by entry distance (node_fast's has a margin); popped entries
+// farther than the current hit are skipped.
 // Candidates win on smaller t, ties on the smaller (instance, primitive) key,
 // so the result does not depend on visit order.
 #pragma once
@@ -255,13 +255,14 @@ struct Tracer {
   // two distances.  Rounding: with u = 2^-24, the reciprocal is off by 2 u,
   // o * inv by u, the offset's sum and the fma by u each, so a distance is
   // off by less than 6 u (|o inv| + |plane inv - o inv|).  The offsets move
-  // every plane outward by 8 u |o inv| and the far distance grows by 32 u of
-  // itself, which also covers the exact test's own rounding: the children
-  // taken are those of the exact test, and now and then one more, whose
-  // primitives cannot win a closer hit.  An entry on the stack is compared
-  // with the hit found meanwhile: its distance may lie 6 u of itself above a
-  // primitive's in the same plane, so the hit's distance grows by the same
-  // 32 u there too (cull).  Empty slots (inf planes) always
+  // every plane outward by 8 u |o inv| and the entry distance shrinks by 32 u
+  // of itself, which also covers the exact test's own rounding: the children
+  // taken are those of the exact test, and now and then one more, which holds
+  // a nearer hit only where a primitive's own distance is rounded further than
+  // its box.  The shrunk entry distance goes on the stack, where it is compared
+  // with the hit found meanwhile: without the margin (it stood on the exit
+  // distance once) it may lie a few u above a primitive's in the same plane,
+  // and equal hits were lost.  Empty slots (inf planes) always
   // fail, or, for a ray of NaNs, lead to a leaf of no primitives.
   //
   // Sorted by a network of five exchanges, reference and distance stored
@@ -300,11 +301,11 @@ struct Tracer {
     }
     const float lo = node_dist(tmin), hi = node_dist(h.t);
     auto slab = [&](float ax, float bx, float ay, float by, float az, float bz) {
-      const float tn = fmaxf(fmaxf(fmaxf(__builtin_fmaf(ax, finv.x, nb.x), __builtin_fmaf(ay, finv.y, nb.y)),
-                                   __builtin_fmaf(az, finv.z, nb.z)), lo);
-      float tf = fminf(fminf(fminf(__builtin_fmaf(bx, finv.x, fb.x), __builtin_fmaf(by, finv.y, fb.y)),
-                             __builtin_fmaf(bz, finv.z, fb.z)), hi);
-      tf = __builtin_fmaf(fabsf(tf), 0x1p-19f, tf);
+      float tn = fmaxf(fmaxf(fmaxf(__builtin_fmaf(ax, finv.x, nb.x), __builtin_fmaf(ay, finv.y, nb.y)),
+                             __builtin_fmaf(az, finv.z, nb.z)), lo);
+      const float tf = fminf(fminf(fminf(__builtin_fmaf(bx, finv.x, fb.x), __builtin_fmaf(by, finv.y, fb.y)),
+                                   __builtin_fmaf(bz, finv.z, fb.z)), hi);
+      tn = __builtin_fmaf(fabsf(tn), -0x1p-19f, tn);
       return tn <= tf ? tn : FINF;
     };
     float t0 = slab(nx.x, fx.x, ny.x, fy.x, nz.x, fz.x), t1 = slab(nx.y, fx.y, ny.y, fy.y, nz.y, fz.y);
@@ -335,13 +336,6 @@ struct Tracer {
       node_base = base;
   }
 
-  // an entry this far away holds nothing nearer than, or as near as, the hit
-  PTD bool cull(float etn) const {
-    if (!FAST) return etn > h.t;
-    const float t = node_dist(h.t);
-    return etn > __builtin_fmaf(fabsf(t), 0x1p-19f, t);
-  }
-
   PTD bool at_node() const { return have && !(ref & LEAF_BIT); }
 
   // the entry in hand, from the stack when there is none; false: the ray is
@@ -360,7 +354,7 @@ struct Tracer {
       if (st.sp == 0) return false;
       float etn;
       st.pop(ref, etn);
-      have = !cull(etn);
+      have = !(etn > (FAST ? node_dist(h.t) : h.t));
     }
     return true;
   }
