@@ -449,7 +449,14 @@ pt_status pt_trace_closest_device(struct pt_context* ctx, const pt_ray* d_rays,
 pt_status pt_trace_closest_device_noalloc(struct pt_context* ctx, const pt_ray* d_rays, uint64_t n,
                                           pt_hit* d_hits, uint32_t* d_overflow_or_null);
 /* Counted variant: per-ray node, primitive and instance fetch counts
- * (3 uint32 per ray), host arrays. */
+ * (3 uint32 per ray), host arrays.  It tests nodes exactly as its counts are
+ * defined; the other entry points (and renders without
+ * PT_FLAG_COUNT_TRAVERSAL) test them conservatively and may visit a few more.
+ * Where a primitive's own distance is rounded further than its box (a sphere
+ * much larger or nearer than its distance, a ray from many scene sizes away,
+ * a negative tmin) they can so find a nearer or equal hit that the exact test
+ * passes by, never a farther one: about one path in 10^9 of the sphere
+ * scene. */
 pt_status pt_trace_closest_counted(struct pt_context* ctx, const pt_ray* rays,
                                    uint64_t n, pt_hit* hits, uint32_t* counts);
 

@@ -67,7 +67,6 @@ PTD float min_component(v3 a) { return ffmin(ffmin(a.x, a.y), a.z); }
 PTD float clampf(float x, float lo, float hi) { return fmaxf(lo, fminf(x, hi)); }
 PTD v3 clamp3(v3 v, float lo, float hi) { return {clampf(v.x, lo, hi), clampf(v.y, lo, hi), clampf(v.z, lo, hi)}; }
 PTD v3 reflect(v3 i, v3 n) { return i - n * (2.0f * dot(n, i)); }
-PTD float comp(v3 v, int k) { return k == 0 ? v.x : (k == 1 ? v.y : v.z); }
 
 // ------------------------------------------------------------------ RNG
 // programs/random.cuh:33-47.  Fully unrolled so that every v + s0 is one add

@@ -40,15 +40,14 @@ constexpr uint32_t EMPTY_CHILD = 0xFFFFFFFFu;
 //   bottom-level structure)
 constexpr int INST_WORDS = 32;
 
-// Block size of the path kernels and the traversal stack: STK_LDS entries per
-// lane in LDS, STK_SPILL more per thread in HBM.
+// Block size of the path kernels and the traversal stack: STK_LDS (queries),
+// STK_LDS_EXTEND or 12 (closest hits) or STK_LDS_SHADE entries per lane in LDS.
 constexpr int BLOCK = 256;
 constexpr int STK_LDS = 16;
 constexpr int STK_LDS_SHADE = 12;  // shading kernel (shadow rays)
 // every thread owns STK_TOTAL entries in all: the ones beyond its kernel's
 // LDS entries spill to its HBM slice of STK_TOTAL entries
 constexpr int STK_TOTAL = 64;
-constexpr int STK_SPILL = STK_TOTAL - STK_LDS;
 // buckets per guide table of the environment sampler's searches
 constexpr uint32_t ENV_GUIDE = 64;
 // closest-hit kernel (k_extend): LDS entries per lane in scenes with meshes,
