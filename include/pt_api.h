@@ -455,8 +455,7 @@ pt_status pt_trace_closest_device_noalloc(struct pt_context* ctx, const pt_ray* 
  * Where a primitive's own distance is rounded further than its box (a sphere
  * much larger or nearer than its distance, a ray from many scene sizes away,
  * a negative tmin) they can so find a nearer or equal hit that the exact test
- * passes by, never a farther one: about one path in 10^9 of the sphere
- * scene. */
+ * passes by, never a farther one: a few paths in 10^9 of the sphere scene. */
 pt_status pt_trace_closest_counted(struct pt_context* ctx, const pt_ray* rays,
                                    uint64_t n, pt_hit* hits, uint32_t* counts);
 

@@ -233,8 +233,9 @@ PTD bool scatter_and_roulette(const Surface& f, v3 Wo, v3 N, uint32_t& seed, uin
 // to state set `out`; finished paths write their slot's result.
 // FEAT: SH_COUNT counts the shadow rays' traversal, SH_CACHE records
 // radiance-cache training vertices and queries, SH_ENV samples environment
-// lights, SH_EXT traces shadow rays through volumes; each is compiled only
-// into the variants that use it.
+// lights, SH_EXT traces shadow rays through volumes, SH_WIDE takes 64-bit node
+// addresses (one scene of 4 GB of nodes or more); each is compiled only into
+// the variants that use it.
 //
 // SH_TAIL (depth0 >= 1 and beyond the cache's query depth, in == src): the launch runs every bounce that is
 // left.  A wave traces the closest hit of its 64 paths itself, shades them,
@@ -249,9 +250,8 @@ PTD bool scatter_and_roulette(const Surface& f, v3 Wo, v3 N, uint32_t& seed, uin
 // for bit.  Against a launch per kernel and bounce, the kernels otherwise as
 // they were then: 64x64 Cornell tile 526 -> 339 us, random spheres 4.29 ->
 // 1.9 ms, next-week scene 10.5 -> 4.1 ms, one 1080p frame of the mesh scene
-// 6.0 -> 4.6 ms (257 us, 1.4, 3.4 and 3.4 ms with the traversal and the
-// spread of small batches of today).
-// SH_WIDE: 64-bit node addresses (one scene of 4 GB of nodes or more).
+// 6.0 -> 4.6 ms (270 us, 1.5, 3.5 and 3.4 ms with the traversal and the
+// spread of small batches of today; 7.6 to 13 lanes are busy per instruction).
 constexpr int SH_COUNT = 1, SH_CACHE = 2, SH_ENV = 4, SH_MULTI = 8, SH_EXT = 16, SH_TAIL = 32, SH_WIDE = 64;
 template <int MS, int FEAT, int KINDS = KIND_ALL>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_shade(
